@@ -19,7 +19,7 @@
  * (RNE), shared by dgrad and wgrad: the grads are f32-accumulated products
  * of 16-bit operands, the contract of the reference's hgemm/bgemm
  * (backend/cpu/gemm.c:575-629).  f32 operands and 1-D (vector) cases use
- * the f32 FMA kernel.
+ * the f32 kernels (pgk_gemm_f32).
  */
 #define _POSIX_C_SOURCE 200809L
 #include "internal.h"
@@ -285,20 +285,23 @@ void pgm_matmul_backward(pg_node *n)
         float *a32 = as_f32(a, &oa), *b32 = as_f32(b, &ob);
         if (!a32 || !b32)
             return;
-        for (size_t z = 0; z < B; z++) {
-            const float *gp = (const float *)g->dev + z * M * N;
-            if (ga) {
-                /* dA[i,p] = sum_j g[i,j] B[p,j] */
-                int beta_z = (s.abat || z == 0) ? ba : 1;
-                float *dst = (float *)ga->dev + (s.abat ? z * M * K : 0);
-                const float *bp = b32 + (s.bbat ? z * K * N : 0);
-                pgk_gemm_f32(0, 1, M, K, N, gp, N, 0, bp, N, 0, dst, K, 0, 1, beta_z, st);
-            }
-            if (gb) {
-                int beta_z = (s.bbat || z == 0) ? bbeta : 1;
-                float *dst = (float *)gb->dev + (s.bbat ? z * K * N : 0);
-                const float *ap = a32 + (s.abat ? z * M * K : 0);
-                pgk_gemm_f32(1, 0, K, N, M, ap, K, 0, gp, N, 0, dst, N, 0, 1, beta_z, st);
+        const float *gp = g->dev;
+        if (ga) { /* dA[i,p] = sum_j g[i,j] B[p,j] */
+            const size_t step = s.abat ? 65535 : 1; /* an unbatched A accumulates over the batch */
+            for (size_t z = 0; z < B; z += step)
+                pgk_gemm_f32(0, 1, M, K, N, gp + z * M * N, N, M * N, b32 + (s.bbat ? z * K * N : 0), N,
+                             s.bbat ? K * N : 0, (float *)ga->dev + (s.abat ? z * M * K : 0), K, M * K,
+                             B - z < step ? B - z : step, z && !s.abat ? 1 : ba, st);
+        }
+        if (gb) { /* dB[p,j] = sum_i A[i,p] g[i,j] */
+            if (!s.bbat && B * M <= 0x7fffffff) { /* the batch folds into the reduction (A is batched, or B == 1) */
+                pgk_gemm_f32(1, 0, K, N, B * M, a32, K, 0, gp, N, 0, gb->dev, N, 0, 1, bbeta, st);
+            } else {
+                const size_t step = s.bbat ? 65535 : 1;
+                for (size_t z = 0; z < B; z += step)
+                    pgk_gemm_f32(1, 0, K, N, M, a32 + (s.abat ? z * M * K : 0), K, s.abat ? M * K : 0, gp + z * M * N, N,
+                                 M * N, (float *)gb->dev + (s.bbat ? z * K * N : 0), N, K * N,
+                                 B - z < step ? B - z : step, z && !s.bbat ? 1 : bbeta, st);
             }
         }
         if (oa)

@@ -27,9 +27,6 @@
 // == 0 for a K-contiguous operand) or k-rows (MN-contiguous) are DMA'd from
 // a 16-byte zero page.  Otherwise the host runs the last K % 64 columns as
 // one more launch over zero-padded copies (beta = 1).
-//
-// k_gemm_f32: plain LDS-tiled f32 FMA GEMM with either operand transposed,
-// for f32 matmuls (not on the bf16/f16 hot path).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -935,62 +932,6 @@ __global__ void __launch_bounds__(256) k_zero_rows(float *__restrict__ c, size_t
     }
 }
 
-// ---------------------------------------------------------------- f32 GEMM
-constexpr int FT = 64, FK = 16;
-
-__global__ void __launch_bounds__(256) k_gemm_f32(int ta, int tb, int M, int N, int K, const float *__restrict__ A,
-                                                  size_t lda, size_t sA, const float *__restrict__ B, size_t ldb,
-                                                  size_t sB, float *__restrict__ C, size_t ldc, size_t sC, int beta)
-{
-    __shared__ float As[FK][FT + 1];
-    __shared__ float Bs[FK][FT + 1];
-    const float *Ab = A + (size_t)blockIdx.z * sA;
-    const float *Bb = B + (size_t)blockIdx.z * sB;
-    float *Cb = C + (size_t)blockIdx.z * sC;
-    const int m0 = blockIdx.y * FT, n0 = blockIdx.x * FT;
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += FK) {
-        for (int q = threadIdx.x; q < FK * FT; q += 256) {
-            int kk = q / FT, mm = q % FT;
-            int gi = m0 + mm, gk = k0 + kk;
-            As[kk][mm] = (gi < M && gk < K) ? (ta ? Ab[(size_t)gk * lda + gi] : Ab[(size_t)gi * lda + gk]) : 0.0f;
-            int gj = n0 + mm;
-            Bs[kk][mm] = (gj < N && gk < K) ? (tb ? Bb[(size_t)gj * ldb + gk] : Bb[(size_t)gk * ldb + gj]) : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < FK; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                a[u] = As[kk][ty * 4 + u];
-                b[u] = Bs[kk][tx * 4 + u];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    acc[u][v] += a[u] * b[v];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        int gi = m0 + ty * 4 + u;
-        if (gi >= M)
-            continue;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            int gj = n0 + tx * 4 + v;
-            if (gj < N) {
-                float *p = Cb + (size_t)gi * ldc + gj;
-                *p = beta ? *p + acc[u][v] : acc[u][v];
-            }
-        }
-    }
-}
-
 struct gemm_args {
     const uint16_t *a;
     size_t lda, sa;
@@ -1518,20 +1459,6 @@ extern "C" int pgk_gemm16_pair_dw(int dtype, const pgk_gemm_desc *d, const pgk_g
     const splitk_desc s1 = pd.sp > 1 ? splitk_of(part_d, pd.sp, d->m, d->n, d->c, d->ldc, d->beta) : splitk_desc{};
     const splitk_desc s2 = pw.sp > 1 ? splitk_of(part_w, pw.sp, w->m, w->n, w->c, w->ldc, w->beta) : splitk_desc{};
     hipLaunchKernelGGL(k_splitk_sum, splitk_grid(s1, s2), dim3(256), 0, st, s1, s2);
-    return (int)hipGetLastError();
-}
-
-extern "C" int pgk_gemm_f32(int ta, int tb, size_t m, size_t n, size_t k, const float *a, size_t lda,
-                            size_t stride_a, const float *b, size_t ldb, size_t stride_b, float *c, size_t ldc,
-                            size_t stride_c, size_t batch, int beta, pgk_stream s)
-{
-    if (!m || !n || !batch)
-        return 0;
-    if (batch > 65535 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff)
-        return (int)hipErrorInvalidValue;
-    dim3 grid((unsigned)((n + FT - 1) / FT), (unsigned)((m + FT - 1) / FT), (unsigned)batch);
-    hipLaunchKernelGGL(k_gemm_f32, grid, dim3(256), 0, (hipStream_t)s, ta, tb, (int)m, (int)n, (int)k, a, lda,
-                       stride_a, b, ldb, stride_b, c, ldc, stride_c, beta);
     return (int)hipGetLastError();
 }
 

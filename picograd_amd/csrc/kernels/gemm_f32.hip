@@ -1,0 +1,451 @@
+// f32 GEMM kernels for gfx950: C[b][i, j] (beta ? += : =) sum_p A(i, p) B(p, j)
+// with f32 operands, f32 products and f32 accumulation on the matrix cores
+// (v_mfma_f32_32x32x2_f32: 256 FLOP per clock and CU, twice what unpacked
+// vector FMAs reach).  Each operand is "K-contiguous" (its reduction dim is
+// contiguous: p[row * ld + k]) or "MN-contiguous" (p[k * ld + row]), at any
+// leading dim and 4-byte alignment.
+//
+// The MFMA takes one k from each half of the wave, and which k is the
+// program's choice as long as A and B agree: lane half h holds the four
+// consecutive k at 8 g + 4 h, so a 32-row fragment of an 8-deep k group is
+// one 16-byte read per lane and feeds four MFMAs.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "launch.h"
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// one problem as the kernels read it
+struct f32_args {
+    const float *a;
+    size_t lda, sa;
+    const float *b;
+    size_t ldb, sb;
+    float *c;
+    size_t ldc, sc;
+    int m, n, k, beta, tiles_n;
+    int va, vb; // 16-byte loads along k (K-contiguous operands)
+};
+
+// block id -> tile: ids are dealt to the 8 XCDs round-robin, so consecutive
+// tiles (which share operand panels) are regrouped onto one XCD and its L2
+__device__ __forceinline__ int xcd_tile(int pid, int nb)
+{
+    return (nb & 7) == 0 ? (pid & 7) * (nb >> 3) + (pid >> 3) : pid;
+}
+
+// the four k values at k .. k + 3 of row `row` (in range); those at or past
+// kend read zero
+template <bool MN>
+__device__ __forceinline__ f32x4 load_k4(const float *__restrict__ p, size_t ld, int row, int k, int kend, bool vec)
+{
+    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (MN) {
+        const float *q = p + (size_t)k * ld + row;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (j < kend - k)
+                v[j] = q[(size_t)j * ld];
+    } else {
+        const float *q = p + (size_t)row * ld + k;
+        if (vec && 3 < kend - k)
+            return *(const f32x4 *)q;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (j < kend - k)
+                v[j] = q[j];
+    }
+    return v;
+}
+
+// the same four values when they are known to lie below kend
+template <bool MN>
+__device__ __forceinline__ f32x4 load_k4_full(const float *__restrict__ p, size_t ld, int row, int k, bool vec)
+{
+    if constexpr (MN) {
+        const float *q = p + (size_t)k * ld + row;
+        return f32x4{q[0], q[ld], q[2 * ld], q[3 * ld]};
+    } else {
+        const float *q = p + (size_t)row * ld + k;
+        if (vec)
+            return *(const f32x4 *)q;
+        return f32x4{q[0], q[1], q[2], q[3]};
+    }
+}
+
+__device__ __forceinline__ f32x16 mfma_f32(float a, float b, const f32x16 &c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
+// Tiled kernel: a block of WGM x WGN waves owns BM x BN of C, each wave
+// (BM / WGM) x (BN / WGN) of it.  K-tiles of KB go global -> registers ->
+// LDS, the next tile's loads in flight while the current one is computed,
+// two LDS buffers and one barrier per tile.  In LDS a tile is
+// [KB / 4][ROWS + 1] slots of four consecutive k of one row: fragment reads
+// are 16 bytes per lane over consecutive rows (no bank conflicts).  Whole
+// tiles load from a wave-uniform base plus a fixed 32-bit offset per lane,
+// so the loop spends no vector ALU work on addresses; an MN-contiguous
+// operand comes as 4 x 4 blocks (four 16-byte loads) transposed in registers,
+// or with 4-byte loads when it is not 16-byte aligned.  Bound by the matrix
+// cores: 4096^3 runs at 121 - 133 TFLOP/s of 157 (128 x 128 tiles), and
+// 2048 x 1024 x 1024 in 44 - 50 us on 64 x 64 tiles (two blocks per CU), where
+// the 64 x 64 vector-FMA kernel before it took 206 - 210 us.
+template <int ROWS, int KB, int NT, bool MN, bool VEC>
+struct F32Tile {
+    static constexpr int KQ = KB / 4, NL = ROWS * KQ / NT, SLOTS = KQ * (ROWS + 1);
+    static_assert(ROWS * KQ % NT == 0, "tile slots divide by the thread count");
+    static constexpr bool BLK = MN && VEC; // 4 x 4 blocks
+    static_assert(!BLK || NL % 4 == 0, "whole 4 x 4 blocks");
+    uint32_t off[NL];
+    // the slot that load q of this thread fills.  BLK: load q reads k row
+    // 4 kq + q % 4 of the four C rows row & ~3 .. row | 3, and after the
+    // transpose slot q % 4 of the block is C row `row`
+    __device__ __forceinline__ static void at(int q, int tid, int &row, int &kq)
+    {
+        if (BLK) {
+            const int i = (q >> 2) * NT + tid;
+            row = i % (ROWS / 4) * 4 + (q & 3);
+            kq = i / (ROWS / 4);
+        } else if (MN) {
+            const int i = q * NT + tid;
+            row = i % ROWS;
+            kq = i / ROWS;
+        } else {
+            const int i = q * NT + tid;
+            row = i / KQ;
+            kq = i % KQ;
+        }
+    }
+    // rows past `extent` read row 0 of the tile (their results are never
+    // stored); BLK has extent % 4 == 0, so a block is wholly in or out
+    __device__ __forceinline__ void init(size_t ld, int row0, int extent, int tid)
+    {
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            int row, kq;
+            at(q, tid, row, kq);
+            if (BLK)
+                off[q] = (uint32_t)(4 * kq + (q & 3)) * (uint32_t)ld * 4 + (row0 + (row & ~3) < extent ? row & ~3 : 0) * 4;
+            else if (MN)
+                off[q] = (uint32_t)(4 * kq) * (uint32_t)ld * 4 + (row0 + row < extent ? row : 0) * 4;
+            else
+                off[q] = (uint32_t)(row0 + row < extent ? row : 0) * (uint32_t)ld * 4 + 16 * kq;
+        }
+    }
+    // a tile wholly below k
+    __device__ __forceinline__ void load_fast(f32x4 (&r)[NL], const float *__restrict__ p, size_t ld, int row0,
+                                              int k0) const
+    {
+        const char *base = (const char *)(MN ? p + (size_t)k0 * ld + row0 : p + (size_t)row0 * ld + k0);
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            if (VEC) {
+                r[q] = *(const f32x4 *)(base + off[q]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    r[q][j] = *(const float *)(base + (MN ? (size_t)j * ld * 4 : (size_t)j * 4) + off[q]);
+            }
+        }
+    }
+    // any tile: values at or past k read zero
+    __device__ __forceinline__ static void load(f32x4 (&r)[NL], const float *__restrict__ p, size_t ld, int row0,
+                                                int extent, int k0, int k, int tid)
+    {
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            int row, kq;
+            at(q, tid, row, kq);
+            if (BLK) {
+                const int kk = k0 + 4 * kq + (q & 3), gr = row0 + (row & ~3) < extent ? row0 + (row & ~3) : row0;
+                r[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (kk < k)
+                    r[q] = *(const f32x4 *)(p + (size_t)kk * ld + gr);
+            } else {
+                r[q] = load_k4<MN>(p, ld, row0 + row < extent ? row0 + row : row0, k0 + 4 * kq, k, VEC);
+            }
+        }
+    }
+    __device__ __forceinline__ static void store(const f32x4 (&r)[NL], f32x4 *lds, int tid)
+    {
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            int row, kq;
+            at(q, tid, row, kq);
+            const int b = q & ~3, i = q & 3;
+            if constexpr (BLK)
+                lds[kq * (ROWS + 1) + pos(row)] = f32x4{r[b][i], r[b + 1][i], r[b + 2][i], r[b + 3][i]};
+            else
+                lds[kq * (ROWS + 1) + row] = r[q];
+        }
+    }
+    // place of a row within its slot row: a 4 x 4 block's writes are 64 bytes
+    // apart, so every other 16 rows take another order of their fours
+    __device__ __forceinline__ static int pos(int row) { return BLK ? row ^ ((row >> 4) & 3) : row; }
+    // rows r0 .. r0 + 31 of the k group at slot row 2 g
+    __device__ __forceinline__ static f32x4 frag(const f32x4 *lds, int r0, int g, int lane)
+    {
+        return lds[(2 * g + (lane >> 5)) * (ROWS + 1) + pos(r0 + (lane & 31))];
+    }
+};
+
+template <int BM, int BN, int WGM, int WGN, int KB, bool TA, bool TB, bool VEC>
+__global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_f32(f32_args g)
+{
+    constexpr int NT = 64 * WGM * WGN, FM = BM / WGM / 32, FN = BN / WGN / 32, KS = KB / 8;
+    using OA = F32Tile<BM, KB, NT, TA, VEC>;
+    using OB = F32Tile<BN, KB, NT, !TB, VEC>;
+    __shared__ f32x4 sa[2][OA::SLOTS], sb[2][OB::SLOTS];
+    const float *__restrict__ A = g.a + (size_t)blockIdx.z * g.sa;
+    const float *__restrict__ B = g.b + (size_t)blockIdx.z * g.sb;
+    float *__restrict__ C = g.c + (size_t)blockIdx.z * g.sc;
+    const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    const int m0 = tile / g.tiles_n * BM, n0 = tile % g.tiles_n * BN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave / WGN * (BM / WGM), wn = wave % WGN * (BN / WGN);
+    f32x16 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                acc[i][j][e] = 0.0f;
+    OA ta;
+    OB tb;
+    ta.init(g.lda, m0, g.m, tid);
+    tb.init(g.ldb, n0, g.n, tid);
+    f32x4 ra[OA::NL], rb[OB::NL];
+    const int kt = g.k / KB + (g.k % KB != 0);
+    auto store = [&](int buf) {
+        OA::store(ra, sa[buf], tid);
+        OB::store(rb, sb[buf], tid);
+    };
+    auto load = [&](int t) {
+        OA::load(ra, A, g.lda, m0, g.m, t * KB, g.k, tid);
+        OB::load(rb, B, g.ldb, n0, g.n, t * KB, g.k, tid);
+    };
+    auto compute = [&](const f32x4 *ca, const f32x4 *cb, int s0, int s1) {
+#pragma unroll
+        for (int s = s0; s < s1; ++s) {
+            f32x4 fa[FM], fb[FN];
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                fa[i] = OA::frag(ca, wm + 32 * i, s, lane);
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                fb[j] = OB::frag(cb, wn + 32 * j, s, lane);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+                        acc[i][j] = mfma_f32(fa[i][q], fb[j][q], acc[i][j]);
+        }
+    };
+    if (kt) {
+        load(0);
+        store(0);
+        __syncthreads();
+    }
+    // tiles whose successor lies wholly below k (32-bit lane offsets reach it
+    // for leading dims under 2^22): no branch in the loop
+    const int fast = g.lda < ((size_t)1 << 22) && g.ldb < ((size_t)1 << 22) ? g.k / KB - 1 : 0;
+    int t = 0;
+    for (; t < fast; ++t) {
+        ta.load_fast(ra, A, g.lda, m0, (t + 1) * KB);
+        tb.load_fast(rb, B, g.ldb, n0, (t + 1) * KB);
+        compute(sa[t & 1], sb[t & 1], 0, KS * 3 / 4);
+        store((t + 1) & 1);
+        compute(sa[t & 1], sb[t & 1], KS * 3 / 4, KS);
+        __syncthreads();
+    }
+    for (; t < kt; ++t) {
+        if (t + 1 < kt)
+            load(t + 1);
+        compute(sa[t & 1], sb[t & 1], 0, KS);
+        if (t + 1 < kt)
+            store((t + 1) & 1);
+        __syncthreads();
+    }
+    // lane holds column lane % 32 of rows 8 (e / 4) + 4 (lane / 32) + e % 4
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            const int col = n0 + wn + 32 * j + (lane & 31);
+            if (col >= g.n)
+                continue;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = m0 + wm + 32 * i + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+                if (row < g.m) {
+                    float *p = C + (size_t)row * g.ldc + col;
+                    *p = g.beta ? *p + acc[i][j][e] : acc[i][j][e];
+                }
+            }
+        }
+}
+
+// Small outputs: a block owns one 32 x 32 tile of C and its eight waves split
+// the reduction, each streaming its k range from global memory straight into
+// MFMA operands (no LDS, no barrier in the k-loop; 32 k in flight ahead of
+// the MFMAs).  The waves' partial tiles are added through LDS in wave order.
+// For outputs with too few 64 x 64 tiles for the chip, where one wave's serial
+// reduction would be the whole time: 256 x 784 x 512 takes 11 us, against
+// 24 - 28 us on 64 x 64 tiles and 103 us for the vector-FMA kernel before it.
+constexpr int kSmWaves = 8, kSmUnroll = 4;
+
+template <bool TA, bool TB>
+__global__ void __launch_bounds__(64 * kSmWaves) k_gemm_f32_small(f32_args g)
+{
+    __shared__ float part[kSmWaves][32][33];
+    const float *__restrict__ A = g.a + (size_t)blockIdx.z * g.sa;
+    const float *__restrict__ B = g.b + (size_t)blockIdx.z * g.sb;
+    float *__restrict__ C = g.c + (size_t)blockIdx.z * g.sc;
+    const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    const int m0 = tile / g.tiles_n * 32, n0 = tile % g.tiles_n * 32;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // this wave's k range, whole groups of 8
+    const int kw = g.k ? (g.k - 1) / (8 * kSmWaves) * 8 + 8 : 0;
+    const int kb = wave * kw < g.k ? wave * kw : g.k;
+    const int kend = g.k - kb > kw ? kb + kw : g.k;
+    const int row = m0 + (lane & 31) < g.m ? m0 + (lane & 31) : g.m - 1;
+    const int col = n0 + (lane & 31) < g.n ? n0 + (lane & 31) : g.n - 1;
+    const int kh = 4 * (lane >> 5);
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+        acc[e] = 0.0f;
+    auto mm = [&](const f32x4 &x, const f32x4 &y) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            acc = mfma_f32(x[q], y[q], acc);
+    };
+    constexpr int U = kSmUnroll;
+    const int whole = kb + (kend - kb) / (8 * U) * (8 * U);
+    f32x4 fa[2][U], fb[2][U];
+    auto load = [&](int buf, int k) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            fa[buf][u] = load_k4_full<TA>(A, g.lda, row, k + 8 * u + kh, g.va);
+            fb[buf][u] = load_k4_full<!TB>(B, g.ldb, col, k + 8 * u + kh, g.vb);
+        }
+    };
+    int k = kb;
+    if (k < whole) {
+        load(0, k);
+        for (; whole - k >= 16 * U; k += 16 * U) {
+            load(1, k + 8 * U);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                mm(fa[0][u], fb[0][u]);
+            if (whole - k > 16 * U)
+                load(0, k + 16 * U);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                mm(fa[1][u], fb[1][u]);
+        }
+        if (k < whole) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                mm(fa[0][u], fb[0][u]);
+            k += 8 * U;
+        }
+    }
+    for (; k < kend; k += 8)
+        mm(load_k4<TA>(A, g.lda, row, k + kh, kend, g.va), load_k4<!TB>(B, g.ldb, col, k + kh, kend, g.vb));
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+        part[wave][(e >> 2) * 8 + (lane >> 5) * 4 + (e & 3)][lane & 31] = acc[e];
+    __syncthreads();
+    const int c = tid & 31;
+    if (n0 + c >= g.n)
+        return;
+#pragma unroll
+    for (int u = 0; u < 1024 / (64 * kSmWaves); ++u) {
+        const int r = (tid >> 5) + u * (2 * kSmWaves);
+        if (m0 + r >= g.m)
+            continue;
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kSmWaves; ++w)
+            v += part[w][r][c];
+        float *p = C + (size_t)(m0 + r) * g.ldc + n0 + c;
+        *p = g.beta ? *p + v : v;
+    }
+}
+
+template <int BM, int BN, int WGM, int WGN, int KB, bool VEC>
+void launch_tiled_v(int ta, int tb, const f32_args &g, dim3 grid, hipStream_t s)
+{
+    const dim3 block(64 * WGM * WGN);
+    switch ((ta ? 2 : 0) | (tb ? 1 : 0)) {
+    case 0: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, false, false, VEC>), grid, block, 0, s, g); break;
+    case 1: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, false, true, VEC>), grid, block, 0, s, g); break;
+    case 2: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, true, false, VEC>), grid, block, 0, s, g); break;
+    default: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, true, true, VEC>), grid, block, 0, s, g); break;
+    }
+}
+
+template <int BM, int BN, int WGM, int WGN, int KB>
+void launch_tiled(int ta, int tb, f32_args g, unsigned batch, hipStream_t s)
+{
+    g.tiles_n = (g.n + BN - 1) / BN;
+    const dim3 grid((unsigned)((g.m + BM - 1) / BM) * (unsigned)g.tiles_n, 1, batch);
+    if (g.va && g.vb)
+        launch_tiled_v<BM, BN, WGM, WGN, KB, true>(ta, tb, g, grid, s);
+    else
+        launch_tiled_v<BM, BN, WGM, WGN, KB, false>(ta, tb, g, grid, s);
+}
+
+void launch_small(int ta, int tb, f32_args g, unsigned batch, hipStream_t s)
+{
+    g.tiles_n = (g.n + 31) / 32;
+    const dim3 grid((unsigned)((g.m + 31) / 32) * (unsigned)g.tiles_n, 1, batch), block(64 * kSmWaves);
+    switch ((ta ? 2 : 0) | (tb ? 1 : 0)) {
+    case 0: hipLaunchKernelGGL((k_gemm_f32_small<false, false>), grid, block, 0, s, g); break;
+    case 1: hipLaunchKernelGGL((k_gemm_f32_small<false, true>), grid, block, 0, s, g); break;
+    case 2: hipLaunchKernelGGL((k_gemm_f32_small<true, false>), grid, block, 0, s, g); break;
+    default: hipLaunchKernelGGL((k_gemm_f32_small<true, true>), grid, block, 0, s, g); break;
+    }
+}
+
+} // namespace
+
+extern "C" int pgk_gemm_f32(int ta, int tb, size_t m, size_t n, size_t k, const float *a, size_t lda,
+                            size_t stride_a, const float *b, size_t ldb, size_t stride_b, float *c, size_t ldc,
+                            size_t stride_c, size_t batch, int beta, pgk_stream s)
+{
+    if (!m || !n || !batch)
+        return 0;
+    if (batch > 65535 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff)
+        return (int)hipErrorInvalidValue;
+    const int va = !(((uintptr_t)a & 15) | (lda & 3) | (stride_a & 3) | (ta ? m & 3 : 0));
+    const int vb = !(((uintptr_t)b & 15) | (ldb & 3) | (stride_b & 3) | (tb ? 0 : n & 3));
+    const f32_args g = {a, lda, stride_a, b, ldb, stride_b, c, ldc, stride_c, (int)m, (int)n, (int)k, beta, 0, va, vb};
+    // the shortest of three plans: rounds of two blocks per CU, a round of
+    // 512 blocks and one of at most 256 (one per CU, which runs a block
+    // faster but leaves the CU short of waves), in units of 39 us at k = 1024.
+    // Measured there: 128 x 128 tiles 137 and 95 us, 64 x 64 tiles 39 and
+    // 33 us, 32 x 32 tiles with the reduction split over the waves 25 and 14 us
+    auto cost = [&](size_t tile, double full, double half) {
+        const size_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * batch, rem = tiles % 512;
+        return (double)(tiles / 512) * full + (rem > 256 ? full : rem ? half : 0.0);
+    };
+    const double big = cost(128, 3.5, 2.4), mid = cost(64, 1.0, 0.85), small = cost(32, 0.64, 0.36);
+    if (small <= mid && small <= big)
+        launch_small(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+    else if (mid <= big)
+        launch_tiled<64, 64, 2, 2, 64>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+    else
+        launch_tiled<128, 128, 2, 2, 32>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+    return (int)hipGetLastError();
+}
