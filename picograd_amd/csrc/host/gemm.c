@@ -153,6 +153,19 @@ static bool pair_full(int dt, const pgk_gemm_desc *dd, const pgk_gemm_desc *dw, 
     return pgd_check(rc, what);
 }
 
+/* The pair in one launch on a split-over-waves tile when both are small
+ * enough to run at once: one launch instead of two, or of split-K's four.
+ * False (nothing launched) otherwise. */
+static bool pair_ks(int dt, const pgk_gemm_desc *dd, const pgk_gemm_desc *dw, const char *what)
+{
+    if (!pgk_gemm16_ks_pair_tile(dd, dw))
+        return false;
+    int tk = pgd_tbegin(PGD_T_GEMM16);
+    int rc = pgk_gemm16_ks_pair(dt, dd, dw, pgd_stream());
+    pgd_tend(tk);
+    return pgd_check(rc, what);
+}
+
 /* 16-bit copy of `rows x cols` (leading dim lds, `batch` matrices `sstride`
  * apart) padded with zeros to rows_pad x cols_pad; src_dtype 0 casts f32 */
 static uint16_t *stage16(int dt, int src_dtype, const void *src, size_t rows, size_t cols, size_t lds,
@@ -352,6 +365,18 @@ void pgm_matmul_backward(pg_node *n)
      * run one after the other on the whole chip. */
     gemm_place pd = PLACE_MAIN, pw = PLACE_MAIN;
     int tk = -1;
+    const pgk_gemm_desc dd = {M, K, N8, g16, N8, M * N8, M, wp, N8, s.bbat ? K * N8 : 0, K, ga ? ga->dev : NULL, K, M * K,
+                              B, ba};
+    const pgk_gemm_desc dw = {K, N, Mw, ap, lda_w, sa_w, lda_w, g16, N8, Mw * N8, N8, gb ? gb->dev : NULL, N,
+                              s.bbat ? K * N : 0, Bw, bbeta};
+    if (d_one && w_one && !alias && pair_ks(dt, &dd, &dw, "dgrad + wgrad")) {
+        if (wpad)
+            pgd_free(wpad, wbytes);
+        if (apad)
+            pgd_free(apad, abytes);
+        pgd_free(g16, gbytes);
+        return;
+    }
     if (d_one && w_one && !alias) {
         double td = pgk_gemm16_time(0, 0, M, K, N8, B, 0), tw = pgk_gemm16_time(1, 1, K, N, Mw, Bw, 0);
         double best = 0.85 * (td + tw);
@@ -369,9 +394,6 @@ void pgm_matmul_backward(pg_node *n)
             pd.timed = pw.timed = false;
             /* one launch holding both when it can (no second stream to
              * fork and join), else the two on two streams */
-            pgk_gemm_desc dd = {M, K, N8, g16, N8, M * N8, M, wp, N8, s.bbat ? K * N8 : 0, K, ga->dev, K, M * K, B, ba};
-            pgk_gemm_desc dw = {K, N, Mw, ap, lda_w, sa_w, lda_w, g16, N8, Mw * N8, N8, gb->dev, N,
-                                s.bbat ? K * N : 0, Bw, bbeta};
             size_t offw = 0, wsz = pgk_gemm16_pair_dw_workspace(&dd, &dw, best_cus, &offw);
             void *ws = wsz ? pgd_scratch(1, wsz) : NULL;
             int rc = wsz && !ws ? PGK_GEMM_NOT_PAIRED : pgk_gemm16_pair_dw(dt, &dd, &dw, best_cus, ws, pgd_stream());
@@ -395,9 +417,6 @@ void pgm_matmul_backward(pg_node *n)
                 pw = (gemm_place){side, 5, 256 - best_cus, false};
             }
         } else {
-            pgk_gemm_desc dd = {M, K, N8, g16, N8, M * N8, M, wp, N8, s.bbat ? K * N8 : 0, K, ga->dev, K, M * K, B, ba};
-            pgk_gemm_desc dw = {K, N, Mw, ap, lda_w, sa_w, lda_w, g16, N8, Mw * N8, N8, gb->dev, N,
-                                s.bbat ? K * N : 0, Bw, bbeta};
             if (pair_full(dt, &dd, &dw, "dgrad + wgrad")) {
                 if (wpad)
                     pgd_free(wpad, wbytes);
@@ -656,7 +675,8 @@ static void mm16_backward(pg_node *n)
     const uint16_t *qa = gb && !alias ? operand16(a, dt, M, K, M, K8, &owna, &oba) : NULL;
     const pgk_gemm_desc dd = {M, K, N8, g16, N8, 0, M, qb, N8, 0, K, ga ? ga->dev : NULL, K, 0, 1, ba};
     const pgk_gemm_desc dw = {K, N, M, qa, K8, 0, K8, g16, N8, 0, N8, gb ? gb->dev : NULL, N, 0, 1, bb};
-    if (!(qb && qa && pair_full(dt, &dd, &dw, "matmul16 dgrad + wgrad"))) {
+    if (!(qb && qa &&
+          (pair_ks(dt, &dd, &dw, "matmul16 dgrad + wgrad") || pair_full(dt, &dd, &dw, "matmul16 dgrad + wgrad")))) {
         if (qb)
             gemm16(dt, 0, 0, M, K, N8, g16, N8, 0, M, qb, N8, 0, K, ga->dev, K, 0, 1, ba, "matmul16 dgrad");
         if (gb && alias)
@@ -968,7 +988,8 @@ void pgm_linear16_backward(pg_node *n)
         narrow_dgrad(px, gx, w, dz16, &dz_owned, dzb, keep ? keep->data_ref : NULL, qw, &ow, obw, M, K, N, N8, dt);
         qw = NULL; /* formed, or pending on gx */
     }
-    if (!(qw && qx && pair_full(dt, &dd, &dw, "linear16 dgrad + wgrad"))) {
+    if (!(qw && qx &&
+          (pair_ks(dt, &dd, &dw, "linear16 dgrad + wgrad") || pair_full(dt, &dd, &dw, "linear16 dgrad + wgrad")))) {
         if (qw)
             gemm16(dt, 0, 0, M, K, N8, dz16, N8, 0, M, qw, N8, 0, K, gx->dev, K, 0, 1, bx, "linear16 dgrad");
         if (gw && alias)

@@ -32,6 +32,7 @@
 
 #include <math.h>
 
+#include <initializer_list>
 #include <type_traits>
 
 #include "convert16.h"
@@ -190,11 +191,15 @@ struct TileMN {
     static constexpr int CPR = ROWS / 8;
     static constexpr int NQ = KB * CPR / NT;
     static_assert(KB * CPR % NT == 0, "tile slots must divide by the thread count");
-    static_assert(CPR >= 16, "the swizzle permutes 16 chunks of a row");
+    static_assert(CPR >= 16 || CPR == 8 || CPR == 4, "the swizzle permutes the 64-byte windows of a row");
     // chunk swizzle of row k: the 64-byte windows of rows k = 0..3 (mod 4)
     // land on four different quarters of the 64 banks, so the 8 rows x 64
-    // bytes one ds_read_b64_tr_b16 touches take the minimum two passes
-    __device__ __forceinline__ static int fk(int k) { return (k & 3) << 2; }
+    // bytes one ds_read_b64_tr_b16 touches take the minimum two passes (two
+    // rows of 128 bytes, or four of 64, already span the banks)
+    __device__ __forceinline__ static int fk(int k)
+    {
+        return CPR >= 16 ? (k & 3) << 2 : CPR == 8 ? (k >> 1 & 1) << 2 : 0;
+    }
 
     // columns past `extent` are clamped to its last 8 (never stored);
     // extent % 8 == 0, extent >= 8
@@ -780,6 +785,198 @@ __global__ void __launch_bounds__(kSkWaves * 64, 1)
     }
 }
 
+// Middle-sized product: a block owns a TM x TN tile of C (32 or 64 a side) and
+// its KG waves split the reduction, wave w taking the KB-deep chunks w,
+// w + KG, ...  Each wave computes the whole tile over its chunks from an
+// S-stage DMA ring of its own, so the k-loop has no block barrier and the
+// waves' load latencies overlap; their partial tiles are then added through
+// LDS in wave order and every thread finishes whole 16-byte pieces of rows
+// (beta, or the forward epilogue).  One launch fills the chip where 128-tiles
+// do not, without split-K's partials in memory and its summing launch.
+// Bound by the loads' latency and the launch itself at these sizes.  Measured
+// back to back against the 128-tile plans (split-K where they split):
+// 512 x 1024 x 4096 dgrad 20.0 -> 14.4 us, 1024^3 20.1 -> 8.4 us, a
+// 512 x 4096 x 1024 gelu layer 22.8 -> 17.1 us, 256 x 256 x 512 9.5 -> 4.5 us.
+template <int TM_, int TN_, int KG_, int KB_, int S_, bool TA_, bool TB_, bool F16_>
+struct kscfg {
+    static constexpr int TM = TM_, TN = TN_, KG = KG_, KB = KB_, S = S_;
+    static constexpr bool TA = TA_, TB = TB_, F16 = F16_;
+    static constexpr int NT = 64 * KG, RS = TN + 4; // floats of a partial tile's row
+    static constexpr int STAGE = (TM + TN) * KB / 8, RING = KG * S * STAGE;
+    static constexpr int PART = KG * TM * RS / 4;
+    static constexpr int LDS_U4 = RING > PART ? RING : PART;
+};
+
+template <class CF>
+__device__ __forceinline__ void ks_block(const gemm_kargs &g, int has_epi, int pid, int nb, bool remap, int z,
+                                         LDS uint4 *const lds)
+{
+    constexpr int TM = CF::TM, TN = CF::TN, KG = CF::KG, KB = CF::KB, S = CF::S, FM = TM / 32, FN = TN / 32;
+    constexpr bool F16 = CF::F16;
+    using OA = typename std::conditional<CF::TA, TileMN<TM, 64, KB>, TileK<TM, 64, KB>>::type;
+    using OB = typename std::conditional<CF::TB, TileMN<TN, 64, KB>, TileK<TN, 64, KB>>::type;
+    constexpr int LPT = OA::NQ + OB::NQ, SA = TM * KB / 8, KS = KB / 16;
+    static_assert((S - 1) * LPT < 64, "the loads in flight fit the vmcnt counter");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // tile order as the tiled kernel's: consecutive tiles on one XCD, 8
+    // tile-rows at a time
+    if (remap && (nb & 7) == 0)
+        pid = (pid & 7) * (nb >> 3) + (pid >> 3);
+    const int group = pid / (8 * g.tiles_n), first = group * 8;
+    const int gsz = g.tiles_m - first < 8 ? g.tiles_m - first : 8, in = pid - group * 8 * g.tiles_n;
+    const int m0 = (first + in % gsz) * TM, n0 = in / gsz * TN;
+    const uint16_t *A = g.A + (size_t)z * g.sA, *B = g.B + (size_t)z * g.sB;
+    LDS uint4 *const ring = lds + wave * S * CF::STAGE;
+    const int nct = (g.K + KB - 1) / KB, nc = nct > wave ? (nct - wave + KG - 1) / KG : 0;
+    const int whole = g.fast_ok ? g.K / KB : 0; // chunks wholly below K
+    typename OA::Fast fA[OA::NQ];
+    typename OB::Fast fB[OB::NQ];
+#pragma unroll
+    for (int q = 0; q < OA::NQ; ++q)
+        fA[q] = OA::fast_q(q, g.lda, m0, g.a_extent, 0, lane);
+#pragma unroll
+    for (int q = 0; q < OB::NQ; ++q)
+        fB[q] = OB::fast_q(q, g.ldb, n0, g.b_extent, 0, lane);
+    // this wave's chunk c into stage st; chunks past the end read the zero page
+    auto load = [&](int c, int st) {
+        LDS uint4 *sa = ring + st * CF::STAGE, *sb = sa + SA;
+        const int ch = c * KG + wave;
+        if (ch < whole) {
+#pragma unroll
+            for (int q = 0; q < OA::NQ; ++q)
+                OA::load_fast(q, fA[q], A, g.lda, m0, ch * KB, sa, 0);
+#pragma unroll
+            for (int q = 0; q < OB::NQ; ++q)
+                OB::load_fast(q, fB[q], B, g.ldb, n0, ch * KB, sb, 0);
+        } else {
+            const int k0 = ch < nct ? ch * KB : g.K;
+#pragma unroll
+            for (int q = 0; q < OA::NQ; ++q)
+                OA::load_q(q, A, g.lda, m0, g.a_extent, k0, g.K, sa, lane);
+#pragma unroll
+            for (int q = 0; q < OB::NQ; ++q)
+                OB::load_q(q, B, g.ldb, n0, g.b_extent, k0, g.K, sb, lane);
+        }
+    };
+    f32x16 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                acc[i][j][e] = 0.0f;
+    if (nc > 0) {
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            load(s, s);
+        int st = 0;
+        for (int c = 0; c < nc; ++c) {
+            const LDS uint4 *sa = ring + st * CF::STAGE, *sb = sa + SA;
+            // chunk c landed (the newest S - 1 chunks may be in flight)
+            __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm((S - 1) * LPT));
+            __asm__ volatile("" ::: "memory");
+            uint4 fa[KS][FM], fb[KS][FN];
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+                    fa[s][i] = OA::frag(sa, i * 32, s, lane);
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    fb[s][j] = OB::frag(sb, j * 32, s, lane);
+            }
+            // the stage's reads are done before its refill
+            __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(63));
+            __asm__ volatile("" ::: "memory");
+            load(c + S, st);
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+                        acc[i][j] = mfma32<F16>(fa[s][i], fb[s][j], acc[i][j]);
+            st = st + 1 == S ? 0 : st + 1;
+        }
+        __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(0));
+    }
+    __syncthreads(); // the rings are done
+    LDS float *part = (LDS float *)lds;
+    const int lrow = lane & 31, lk = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                part[(wave * TM + i * 32 + (e >> 2) * 8 + lk * 4 + (e & 3)) * CF::RS + j * 32 + lrow] = acc[i][j][e];
+    __syncthreads();
+    float *C = g.C + (size_t)z * g.sC;
+    const pgk_epi &epi = g.epi;
+    const bool v4 = (g.ldc & 3) == 0 && (((uintptr_t)C | (uintptr_t)epi.z) & 15) == 0 && (((uintptr_t)epi.c16) & 7) == 0;
+#pragma unroll
+    for (int i = (int)threadIdx.x; i < TM * TN / 4; i += CF::NT) {
+        const int row = i / (TN / 4), c4 = i % (TN / 4) * 4;
+        const int gr = m0 + row, gc = n0 + c4;
+        if (gr >= g.M || gc >= g.N)
+            continue;
+        f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < KG; ++w)
+            v += *(const LDS f32x4 *)(part + (w * TM + row) * CF::RS + c4);
+        const size_t off = (size_t)gr * g.ldc + gc;
+        if (!v4 || gc + 3 >= g.N) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (gc + q >= g.N)
+                    break;
+                if (has_epi)
+                    epi_store(epi, C, off + q, gc + q, v[q]);
+                else
+                    C[off + q] = g.beta ? C[off + q] + v[q] : v[q];
+            }
+        } else if (has_epi) {
+            f32x4 zv = v, o;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                zv[q] += epi.bias ? epi.bias[gc + q] : 0.0f;
+                o[q] = act_f(epi.act, zv[q]);
+            }
+            if (!epi.skip_out)
+                *(f32x4 *)(C + off) = o;
+            if (epi.z)
+                *(f32x4 *)(epi.z + off) = zv;
+            if (epi.c16)
+                *(uint2 *)(epi.c16 + off) = make_uint2(to16x2(epi.dtype16, o[0], o[1]), to16x2(epi.dtype16, o[2], o[3]));
+        } else {
+            *(f32x4 *)(C + off) = g.beta ? *(const f32x4 *)(C + off) + v : v;
+        }
+    }
+}
+
+template <class CF>
+__global__ void __launch_bounds__(CF::NT, 1) k_gemm16_ks(gemm_kargs g, int has_epi)
+{
+    __shared__ uint4 smem[CF::LDS_U4];
+    ks_block<CF>(g, has_epi, (int)blockIdx.x, (int)gridDim.x, true, (int)blockIdx.z, (LDS uint4 *)smem);
+}
+
+// a matmul's dgrad (blocks [0, n1)) and wgrad in one launch, each nb tiles
+// per batch entry, on one tile shape
+template <class C1, class C2>
+__global__ void __launch_bounds__(C1::NT, 1) k_gemm16_ks_pair(gemm_kargs g1, gemm_kargs g2, int nb1, int n1, int nb2)
+{
+    static_assert(C1::NT == C2::NT && C1::LDS_U4 == C2::LDS_U4, "one tile shape");
+    __shared__ uint4 smem[C1::LDS_U4];
+    const int b = (int)blockIdx.x;
+    if (b < n1)
+        ks_block<C1>(g1, 0, b % nb1, nb1, true, b / nb1, (LDS uint4 *)smem);
+    else
+        ks_block<C2>(g2, 0, (b - n1) % nb2, nb2, (n1 & 7) == 0, (b - n1) / nb2, (LDS uint4 *)smem);
+}
+
 // the same epilogue as a pass over a finished C (k-tail runs)
 __global__ void __launch_bounds__(256) k_bias_act(float *__restrict__ c, size_t ldc, int m, int n, pgk_epi epi)
 {
@@ -973,6 +1170,77 @@ int launch_tile(const gemm_args &g, const pgk_epi &epi, hipStream_t s)
     return (int)hipGetLastError();
 }
 
+// the split-over-waves tiles of the planner: 5 is 32 x 32 with eight waves, 6
+// 32 x 64 with eight, 7 64 x 64 with four (two blocks per CU).  Deeper rings
+// and 64 x 64 with eight waves measured slower.
+template <int TILE, bool TA, bool TB, bool F16>
+using ks_cfg = typename std::conditional<
+    TILE == 5, kscfg<32, 32, 8, 64, 2, TA, TB, F16>,
+    typename std::conditional<TILE == 6, kscfg<32, 64, 8, 32, 3, TA, TB, F16>,
+                              kscfg<64, 64, 4, 32, 2, TA, TB, F16>>::type>::type;
+
+template <class CF>
+gemm_kargs ks_kargs(const gemm_args &g, const pgk_epi &epi)
+{
+    return make_kargs<gcfg<CF::TM, CF::TN, 1, 1, CF::TA, CF::TB, CF::F16, false, 64, 2>>(g, epi);
+}
+
+template <class CF>
+int launch_ks(const gemm_args &g, const pgk_epi &epi, int has_epi, hipStream_t s)
+{
+    const gemm_kargs k = ks_kargs<CF>(g, epi);
+    hipLaunchKernelGGL(k_gemm16_ks<CF>, dim3((unsigned)(k.tiles_m * k.tiles_n), 1, g.batch), dim3(CF::NT), 0, s, k,
+                       has_epi);
+    return (int)hipGetLastError();
+}
+
+template <bool TA, bool TB, bool F16>
+int launch_ks_tile(const gemm_args &g, const pgk_epi &epi, int has_epi, hipStream_t s)
+{
+    switch (g.tile) {
+    case 5: return launch_ks<ks_cfg<5, TA, TB, F16>>(g, epi, has_epi, s);
+    case 6: return launch_ks<ks_cfg<6, TA, TB, F16>>(g, epi, has_epi, s);
+    default: return launch_ks<ks_cfg<7, TA, TB, F16>>(g, epi, has_epi, s);
+    }
+}
+
+int launch_ks_any(int f16, int ta, int tb, const gemm_args &g, const pgk_epi &epi, int has_epi, hipStream_t s)
+{
+    const int sel = (f16 ? 4 : 0) | (ta ? 2 : 0) | (tb ? 1 : 0);
+    switch (sel) {
+    case 0: return launch_ks_tile<false, false, false>(g, epi, has_epi, s);
+    case 1: return launch_ks_tile<false, true, false>(g, epi, has_epi, s);
+    case 2: return launch_ks_tile<true, false, false>(g, epi, has_epi, s);
+    case 3: return launch_ks_tile<true, true, false>(g, epi, has_epi, s);
+    case 4: return launch_ks_tile<false, false, true>(g, epi, has_epi, s);
+    case 5: return launch_ks_tile<false, true, true>(g, epi, has_epi, s);
+    case 6: return launch_ks_tile<true, false, true>(g, epi, has_epi, s);
+    default: return launch_ks_tile<true, true, true>(g, epi, has_epi, s);
+    }
+}
+
+template <bool F16, int TILE>
+int launch_ks_pair(const gemm_args &gd, const gemm_args &gw, hipStream_t s)
+{
+    using CD = ks_cfg<TILE, false, false, F16>;
+    using CW = ks_cfg<TILE, true, true, F16>;
+    const gemm_kargs kd = ks_kargs<CD>(gd, pgk_epi{}), kw = ks_kargs<CW>(gw, pgk_epi{});
+    const int nb1 = kd.tiles_m * kd.tiles_n, nb2 = kw.tiles_m * kw.tiles_n;
+    const int n1 = nb1 * (int)gd.batch, n2 = nb2 * (int)gw.batch;
+    hipLaunchKernelGGL((k_gemm16_ks_pair<CD, CW>), dim3((unsigned)(n1 + n2)), dim3(CD::NT), 0, s, kd, kw, nb1, n1, nb2);
+    return (int)hipGetLastError();
+}
+
+template <bool F16>
+int launch_ks_pair_tile(int tile, const gemm_args &gd, const gemm_args &gw, hipStream_t s)
+{
+    switch (tile) {
+    case 5: return launch_ks_pair<F16, 5>(gd, gw, s);
+    case 6: return launch_ks_pair<F16, 6>(gd, gw, s);
+    default: return launch_ks_pair<F16, 7>(gd, gw, s);
+    }
+}
+
 // The configurations launch_layout picks from (the planner's tile ids):
 //  - 2: 256 x 256 tiles, eight waves of 128 x 64; k-tiles of 32 in a
 //    four-stage ring (128 KiB of LDS), except with both operands
@@ -1145,13 +1413,52 @@ __global__ void __launch_bounds__(512, 1) k_mfma_probe(float *sink, int iters, i
 // Ragged shapes such as M = 4097 (33 rows of 128-tiles) and weight grads
 // with a short output dim are where it matters.
 typedef struct {
-    int tile; // 2 = 256 x 256, 3 = 128 x 256, 1 = 128 x 128
+    int tile; // 2 = 256 x 256, 3 = 128 x 256, 1 = 128 x 128, 5 - 7: ks_tile
     int sp;   // split-K factor, 1 = none
 } gemm_plan;
 
 // `cu_budget` is the number of CUs the launch may occupy (another launch
 // runs beside it on the rest), 0 for the whole chip.
 static constexpr int kCUs = 256;
+
+// The split-over-waves tile for `problems` problems run as one launch, 0 when
+// none: the smallest tile whose blocks all run at once, one per CU (two for
+// the 64 x 64 tile).  Each beats the larger ones and the 128-tile plans up to
+// that count at every reduction measured (128 to 4096: 32 x 32 at 256 blocks
+// 3.7 - 13 against 7.2 - 20 us; 64 x 64 at 512 blocks 7.1 - 33 against 7.5 -
+// 36 us); past it they lose (64 x 64 at 1024 blocks 12 - 21 against 7.6 - 17
+// us).  Products of at most 16 columns keep their plans: more than half of
+// these tiles would be padding.
+struct ks_size {
+    size_t m, n, batch;
+};
+static int ks_tile(std::initializer_list<ks_size> problems)
+{
+    static const struct {
+        int tile;
+        size_t tm, tn, most;
+    } shapes[3] = {{5, 32, 32, 256}, {6, 32, 64, 256}, {7, 64, 64, 512}};
+    for (const auto &sh : shapes) {
+        size_t blocks = 0;
+        for (const ks_size &q : problems)
+            blocks += ((q.m + sh.tm - 1) / sh.tm) * ((q.n + sh.tn - 1) / sh.tn) * q.batch;
+        if (blocks <= sh.most)
+            return sh.tile;
+    }
+    return 0;
+}
+
+// its time, from the same measurements: a launch and a rate per k
+static double ks_time(int tile, size_t m, size_t n, size_t k, size_t batch)
+{
+    const double kk = (double)k / 1024.0;
+    if (tile == 5)
+        return (3.4 + 1.8 * kk) * 1e-6;
+    if (tile == 6)
+        return (3.8 + 2.6 * kk) * 1e-6;
+    const size_t blocks = ((m + 63) / 64) * ((n + 63) / 64) * batch;
+    return (blocks <= 256 ? 4.6 + 3.5 * kk : 6.0 + 6.8 * kk) * 1e-6;
+}
 
 // Time model: rounds of one block per CU, each block at its tile's rate
 // per CU (measured under a loaded chip), plus for a split its partials:
@@ -1161,7 +1468,14 @@ static constexpr int kCUs = 256;
 // HBM capacity.
 static gemm_plan plan_gemm(size_t m, size_t n, size_t kin, size_t batch, int cu_budget = 0, double *time = nullptr)
 {
-    const double cus = cu_budget > 0 && cu_budget < kCUs ? (double)cu_budget : (double)kCUs;
+    const bool whole = !(cu_budget > 0 && cu_budget < kCUs);
+    const double cus = whole ? (double)kCUs : (double)cu_budget;
+    const int ks = whole && n > 16 && kin ? ks_tile({{m, n, batch}}) : 0;
+    if (ks) {
+        if (time)
+            *time = ks_time(ks, m, n, kin, batch);
+        return {ks, 1};
+    }
     struct shape {
         int tile;
         size_t bm, bn;
@@ -1338,7 +1652,14 @@ extern "C" int pgk_gemm16_cu(int dtype, int ta, int tb, size_t m, size_t n, size
     // the epilogue rides on the GEMM when one launch of the forward layout
     // finishes C, on the split-K sum when that finishes C, otherwise it is
     // a pass over C afterwards
-    if (has_epi && !sp && !ktail && !ta && tb) {
+    if (pl.tile >= 5 && kmain) {
+        const bool fused = has_epi && !ktail;
+        gemm_args g = {a, lda, stride_a, (int)a_extent, b, ldb, stride_b, (int)b_extent, c, ldc, stride_c,
+                       (int)m, (int)n, (int)kmain, beta, (unsigned)batch, pl.tile};
+        const int rc = launch_ks_any(f16, ta, tb, g, fused ? *epi : pgk_epi{}, fused, st);
+        if (rc || fused || (!ktail && !has_epi))
+            return rc;
+    } else if (has_epi && !sp && !ktail && !ta && tb) {
         gemm_args g = {a, lda, stride_a, (int)a_extent, b, ldb, stride_b, (int)b_extent, c, ldc, stride_c,
                        (int)m, (int)n, (int)kmain, 0, 1u, pl.tile};
         return f16 ? launch_layout<false, true, true, true>(g, st, *epi)
@@ -1348,7 +1669,9 @@ extern "C" int pgk_gemm16_cu(int dtype, int ta, int tb, size_t m, size_t n, size
     if ((sp || ktail) && !ws)
         return (int)hipErrorInvalidValue;
     int rc = 0;
-    if (kmain && sp) {
+    if (pl.tile >= 5) {
+        // queued above; a k tail and its epilogue follow
+    } else if (kmain && sp) {
         // slice z covers k in [z * ks, min(kmain, (z + 1) * ks)): operand
         // offsets along the reduction, dense [m, n] partials
         const size_t ks = ((kmain + sp - 1) / sp + BK - 1) / BK * BK;
@@ -1430,7 +1753,7 @@ extern "C" int pgk_gemm16_pair_dw(int dtype, const pgk_gemm_desc *d, const pgk_g
         return PGK_GEMM_NOT_PAIRED;
     const gemm_plan pd = plan_gemm(d->m, d->n, d->k, d->batch, cu_d), pw = plan_gemm(w->m, w->n, w->k, w->batch,
                                                                                       kCUs - cu_d);
-    if (pd.tile != pw.tile)
+    if (pd.tile != pw.tile || pd.tile >= 5)
         return PGK_GEMM_NOT_PAIRED;
     size_t off_w = 0;
     pgk_gemm16_pair_dw_workspace(d, w, cu_d, &off_w);
@@ -1460,6 +1783,35 @@ extern "C" int pgk_gemm16_pair_dw(int dtype, const pgk_gemm_desc *d, const pgk_g
     const splitk_desc s2 = pw.sp > 1 ? splitk_of(part_w, pw.sp, w->m, w->n, w->c, w->ldc, w->beta) : splitk_desc{};
     hipLaunchKernelGGL(k_splitk_sum, splitk_grid(s1, s2), dim3(256), 0, st, s1, s2);
     return (int)hipGetLastError();
+}
+
+extern "C" int pgk_gemm16_ks_pair_tile(const pgk_gemm_desc *d, const pgk_gemm_desc *w)
+{
+    if (!d->m || !d->n || !d->k || !d->batch || !w->m || !w->n || !w->k || !w->batch || d->k % 8 ||
+        skinny_ok(1, 1, w->m, w->n, w->k, w->batch))
+        return 0;
+    return ks_tile({{d->m, d->n, d->batch}, {w->m, w->n, w->batch}});
+}
+
+extern "C" int pgk_gemm16_ks_pair(int dtype, const pgk_gemm_desc *d, const pgk_gemm_desc *w, pgk_stream s)
+{
+    const int tile = pgk_gemm16_ks_pair_tile(d, w);
+    if (!tile)
+        return PGK_GEMM_NOT_PAIRED;
+    int bad = check_gemm_args(0, 0, d->m, d->n, d->k, d->a, d->lda, d->stride_a, d->a_extent, d->b, d->ldb,
+                              d->stride_b, d->b_extent, d->batch);
+    if (!bad)
+        bad = check_gemm_args(1, 1, w->m, w->n, w->k, w->a, w->lda, w->stride_a, w->a_extent, w->b, w->ldb,
+                              w->stride_b, w->b_extent, w->batch);
+    if (bad)
+        return bad;
+    auto args = [&](const pgk_gemm_desc *x) {
+        return gemm_args{x->a, x->lda, x->stride_a, (int)x->a_extent, x->b, x->ldb, x->stride_b, (int)x->b_extent,
+                         x->c, x->ldc, x->stride_c, (int)x->m, (int)x->n, (int)x->k, x->beta, (unsigned)x->batch, tile};
+    };
+    const gemm_args gd = args(d), gw = args(w);
+    return dtype == 1 ? launch_ks_pair_tile<true>(tile, gd, gw, (hipStream_t)s)
+                      : launch_ks_pair_tile<false>(tile, gd, gw, (hipStream_t)s);
 }
 
 extern "C" int pgk_mfma_probe(int lds, float *sink, size_t sink_floats, int blocks, int iters, pgk_stream s)

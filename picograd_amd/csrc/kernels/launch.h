@@ -190,6 +190,11 @@ typedef struct {
  * pair: a k that needs a zero-padded tail launch, or the plans choose
  * different tile sizes.  ws: pgk_gemm16_pair_dw_workspace bytes. */
 #define PGK_GEMM_NOT_PAIRED (-1)
+/* The same pair in one launch on a split-over-waves tile (pgk_gemm16_plan's
+ * 5 to 7), no workspace; _tile is that tile, 0 when none holds both (the
+ * launch is then refused as PGK_GEMM_NOT_PAIRED). */
+int pgk_gemm16_ks_pair_tile(const pgk_gemm_desc *d, const pgk_gemm_desc *w);
+int pgk_gemm16_ks_pair(int dtype, const pgk_gemm_desc *d, const pgk_gemm_desc *w, pgk_stream s);
 size_t pgk_gemm16_pair_dw_workspace(const pgk_gemm_desc *d, const pgk_gemm_desc *w, int cu_d, size_t *off_w);
 int pgk_gemm16_pair_dw(int dtype, const pgk_gemm_desc *d, const pgk_gemm_desc *w, int cu_d, void *ws,
                        pgk_stream s);
