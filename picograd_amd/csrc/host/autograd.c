@@ -306,11 +306,13 @@ typedef struct {
     int dt16;
 } lz_op;
 
-/* reduce_all over a run's output, recorded with the run when it is small
- * (pgj_small_reduce_fits): both reduction nodes' values come from the run's
- * one-block kernel */
+/* reduce_all over a run's output, recorded with the run.  When it is small
+ * (pgj_small_reduce_fits) both reduction nodes' values come from the run's
+ * one-block kernel; else (wide) the run's kernel also sums the output's
+ * columns, as a fused backward sums a bias grad's, and the column sums are
+ * added by one more launch */
 typedef struct {
-    bool on;
+    bool on, wide;
     int src; /* op index whose output is reduced */
     lz_tensor r1, r2;
     float scale;
@@ -440,7 +442,7 @@ static bool lz_run_eager(int k)
 static bool lz_run_small(pg_jit_graph *g, const void *const *x_in, size_t nx_in, void *const *x_out, size_t nx_out)
 {
     size_t numel = pg_shape_numel(g_lz.ndim, g_lz.shape);
-    if (numel > PGJ_SMALL_MAX)
+    if (numel > PGJ_SMALL_MAX || (g_lz.red.on && g_lz.red.wide))
         return false;
     if (g_lz.red.on && !pgj_small_reduce_fits(g_lz.ndim, g_lz.shape))
         return false;
@@ -502,13 +504,39 @@ static pg_jit_graph *lz_graph(int *idi, int *ido)
     return g;
 }
 
+/* the run's own outputs plus, for a wide reduction, its column sums: the
+ * graph gains that output, out[] its address; returns how many were added */
+static size_t lz_mark_wide(pg_jit_graph *g, const int *ido, void **out)
+{
+    if (!g_lz.red.on || !g_lz.red.wide)
+        return 0;
+    pgj_mark_output_ex(g, ido[g_lz.red.src], 1, g_lz.red.r1.shape, 0);
+    out[0] = g_lz.red.r1.dev;
+    return 1;
+}
+
+/* after the kernel that wrote the column sums: their total */
+static bool lz_wide_total(void)
+{
+    return pgd_check(pgk_sum_vec_f32(g_lz.red.r1.dev, g_lz.red.r2.dev, g_lz.red.r1.shape[0], g_lz.red.scale,
+                                     pgd_stream()),
+                     "reduce");
+}
+
 /* the run has executed (or failed with its device error recorded): the
  * recorded reduction falls back to its own launch if the run's kernel did
  * not compute it, and every held reference is released */
 static void lz_finish(bool ran, bool red_done)
 {
     if (g_lz.red.on) {
-        if (!red_done && ran)
+        if (!red_done && ran && g_lz.red.wide) {
+            const size_t wsz = pgk_sum_axis_workspace(1, g_lz.shape[0], g_lz.shape[1]);
+            void *ws = wsz ? pgd_scratch(2, wsz) : NULL;
+            if ((!wsz || ws) && pgd_check(pgk_sum_axis_f32(g_lz.op[g_lz.red.src].out.dev, g_lz.red.r1.dev, 1, g_lz.shape[0],
+                                                           g_lz.shape[1], 1.0f, ws, pgd_stream()),
+                                          "reduce"))
+                lz_wide_total();
+        } else if (!red_done && ran)
             pgd_check(pgk_sum_all2_f32(g_lz.op[g_lz.red.src].out.dev, g_lz.red.r1.dev, g_lz.red.r2.dev,
                                        g_lz.shape[0], g_lz.shape[1], g_lz.red.scale, pgd_stream()),
                       "reduce");
@@ -548,12 +576,12 @@ void pga_lazy_flush(void)
             pgj_mark_output16(g, ido[k], g_lz.op[k].dt16);
             x16[n16++] = g_lz.op[k].out16;
         }
-    if (g && n16) {
+    if (g && (n16 || (g_lz.red.on && g_lz.red.wide))) {
         if (lz_run_small(g, NULL, 0, x16, n16)) {
             ok = red_done = true;
         } else {
             const void *ip[LZ_MAX];
-            void *op[2 * LZ_MAX];
+            void *op[2 * LZ_MAX + 1];
             size_t no = 0;
             for (int j = 0; j < g_lz.nin; j++)
                 ip[j] = g_lz.in[j].dev;
@@ -561,9 +589,11 @@ void pga_lazy_flush(void)
                 op[no++] = g_lz.op[k].out.dev;
             for (size_t k = 0; k < n16; k++)
                 op[no++] = x16[k];
-            ok = pgj_launch(g, g_lz.ndim, g_lz.shape, ip, (size_t)g_lz.nin, op, no);
+            const size_t wide = lz_mark_wide(g, ido, op + no);
+            ok = pgj_launch(g, g_lz.ndim, g_lz.shape, ip, (size_t)g_lz.nin, op, no + wide);
+            red_done = ok && wide && lz_wide_total();
         }
-        g_lz_wrote16 = ok;
+        g_lz_wrote16 = ok && n16;
         pg_jit_graph_free(g);
         g = NULL;
     }
@@ -620,23 +650,27 @@ static bool lz_overlaps_ptr(const lz_tensor *x, const void *p, size_t nbytes)
     return a < b + nbytes && b < a + na;
 }
 
-/* A fused backward region (graph bwd over the loop shape (lnd, ls),
- * inputs bin[], full-shape outputs bout[]) executed in the same one-block
- * kernel as the pending small run, after the run's values in each element
- * (one launch instead of two: config 1's leaves, forward, reduction and
- * backward).  bwd's inputs that are run inputs or outputs read those
- * values; its outputs (the grads) must not overlap the run's tensors.  The
- * merged body is compiled without FMA contraction, as the run is.  True
- * when the merged kernel was launched (the run is then done); false with
- * nothing launched and the run still pending otherwise. */
+/* A fused backward region (graph bwd over the loop shape (lnd, ls), inputs
+ * bin[], outputs bout[]) executed in the pending run's own kernel, after the
+ * run's values in each element: one launch instead of two, and the region
+ * reads the run's operands and values from registers instead of memory
+ * (gelu(x + bias) * sigmoid(g) over [16384, 4096] with its sum and grads,
+ * 2.1 GB in place of 2.9: 600 -> 424 us; [3001, 1037]: 53 -> 35 us).  bwd's inputs that are run inputs or outputs read those
+ * values; its outputs (the grads) must not overlap the run's tensors.  A
+ * small run takes the region into its one block when every grad has the
+ * loop shape, compiled without FMA contraction as the run is; a larger one
+ * takes it into the main kernel, where a grad may also be summed onto
+ * trailing dims and the region's own operations stay contracted.  True when
+ * the merged kernel was launched (the run is then done); false with nothing
+ * launched and the run still pending otherwise. */
 bool pga_lazy_flush_with_backward(const pg_jit_graph *bwd, size_t lnd, const size_t *ls, const void *const *bin,
                                   size_t bnin, void *const *bout, size_t bnout)
 {
-    if (!g_lz.nops || g_lz.flushing || !pg_shape_equal(lnd, ls, g_lz.ndim, g_lz.shape) ||
-        pg_shape_numel(lnd, ls) > PGJ_SMALL_MAX || bnin > 32 || bnout > 32)
+    if (!g_lz.nops || g_lz.flushing || !pg_shape_equal(lnd, ls, g_lz.ndim, g_lz.shape) || bnin > 32 || bnout > 32)
         return false;
-    const size_t obytes = pg_shape_numel(lnd, ls) * 4;
+    const bool small = pg_shape_numel(lnd, ls) <= PGJ_SMALL_MAX;
     for (size_t o = 0; o < bnout; o++) {
+        const size_t obytes = pgj_output_bytes(bwd, o);
         for (int j = 0; j < g_lz.nin; j++)
             if (lz_overlaps_ptr(&g_lz.in[j], bout[o], obytes))
                 return false;
@@ -651,6 +685,12 @@ bool pga_lazy_flush_with_backward(const pg_jit_graph *bwd, size_t lnd, const siz
     pg_jit_graph *g = lz_graph(idi, ido);
     if (!g)
         return false;
+    void *op[2 * LZ_MAX + 32];
+    size_t no = 0;
+    for (int k = 0; k < g_lz.nops; k++)
+        op[no++] = g_lz.op[k].out.dev;
+    const size_t wide = lz_mark_wide(g, ido, op + no);
+    no += wide;
     /* bwd's inputs: a run output or input with the same address and shape,
      * else a new input of the merged kernel (one overlapping a run tensor
      * otherwise cannot be read in the same pass) */
@@ -666,6 +706,10 @@ bool pga_lazy_flush_with_backward(const pg_jit_graph *bwd, size_t lnd, const siz
             break;
         const size_t nb = pg_shape_numel(nd, sh) * 4;
         in_map[i] = -1;
+        if (g_lz.red.on && (lz_overlaps_ptr(&g_lz.red.r1, bin[i], nb) || lz_overlaps_ptr(&g_lz.red.r2, bin[i], nb))) {
+            ok = false;
+            break;
+        }
         for (int k = 0; k < g_lz.nops && in_map[i] < 0 && ok; k++) {
             const lz_tensor *x = &g_lz.op[k].out;
             if (x->dev == bin[i] && pg_shape_equal(x->ndim, x->shape, nd, sh))
@@ -687,26 +731,50 @@ bool pga_lazy_flush_with_backward(const pg_jit_graph *bwd, size_t lnd, const siz
             x_in[nx++] = bin[i];
         }
     }
-    ok = ok && pgj_graph_append(g, bwd, in_map, lnd, ls);
+    ok = ok && pgj_graph_append(g, bwd, in_map, lnd, ls, small);
     if (ok) {
         g_lz.flushing = true;
-        ok = lz_run_small(g, x_in, nx, bout, bnout);
+        if (small && !wide) {
+            ok = lz_run_small(g, x_in, nx, bout, bnout);
+            if (ok)
+                lz_finish(true, true);
+        } else {
+            const void *ip[2 * LZ_MAX + 32];
+            size_t ni = 0;
+            for (int j = 0; j < g_lz.nin; j++)
+                ip[ni++] = g_lz.in[j].dev;
+            for (size_t j = 0; j < nx; j++)
+                ip[ni++] = x_in[j];
+            for (size_t o = 0; o < bnout; o++)
+                op[no++] = bout[o];
+            ok = pgj_launch(g, lnd, ls, ip, ni, op, no);
+            if (ok)
+                lz_finish(true, wide && lz_wide_total());
+        }
         g_lz.flushing = false;
-        if (ok)
-            lz_finish(true, true);
     }
     pg_jit_graph_free(g);
     return ok;
 }
 
+/* the reductions a run's main kernel takes: column sums are its business
+ * with two or more rows and columns, and one block adds up to 64 Ki of them */
+static bool lz_reduces_wide(const pg_tensor *t)
+{
+    return t->ndim == 2 && t->shape[0] > 1 && t->shape[1] > 1 && t->shape[1] <= 65536 &&
+           pg_shape_numel(t->ndim, t->shape) > PGJ_SMALL_MAX;
+}
+
 /* reduce_all's two values from the pending run when t is one of its
- * outputs and the run is small: the reduction is recorded and computed by
- * the run's kernel.  False (nothing recorded) otherwise. */
+ * outputs: the reduction is recorded and computed by the run's kernel.
+ * False (nothing recorded) otherwise. */
 static bool lz_record_reduce_all(const pg_tensor *t, bool mean, pg_tensor **v1, pg_tensor **v2)
 {
     if (!g_lz.nops || g_lz.red.on || g_lz.flushing || !pg_autograd_is_jit_enabled() || t->ndim != 2 ||
-        !pg_shape_equal(t->ndim, t->shape, g_lz.ndim, g_lz.shape) || !pgj_small_reduce_fits(t->ndim, t->shape) ||
-        pg_shape_numel(t->ndim, t->shape) > PGJ_SMALL_MAX)
+        t->dtype != PG_DTYPE_F32 || !pgt_is_contiguous(t) || !pg_shape_equal(t->ndim, t->shape, g_lz.ndim, g_lz.shape))
+        return false;
+    const bool wide = lz_reduces_wide(t);
+    if (!wide && (!pgj_small_reduce_fits(t->ndim, t->shape) || pg_shape_numel(t->ndim, t->shape) > PGJ_SMALL_MAX))
         return false;
     int src = lz_find(t);
     if (src >= 0 || src <= -LZ_MAX - 1)
@@ -723,6 +791,7 @@ static bool lz_record_reduce_all(const pg_tensor *t, bool mean, pg_tensor **v1, 
     g_lz.red.scale = mean ? 1.0f / (float)cols : 1.0f;
     lz_hold(&g_lz.red.r1, (*v1)->data_ref, (*v1)->dev, 1, (*v1)->shape);
     lz_hold(&g_lz.red.r2, (*v2)->data_ref, (*v2)->dev, 1, (*v2)->shape);
+    g_lz.red.wide = wide;
     g_lz.red.on = true;
     return true;
 }
@@ -1122,6 +1191,19 @@ static pg_node *reduce_all(pg_node *a, bool mean)
         pg_node *out = reduce_attach(n1, 0, false, mean, v2);
         pg_node_free(n1);
         return out;
+    }
+    if (lz_reduces_wide(t)) {
+        pg_tensor *v1 = NULL, *v2 = NULL;
+        if (lz_record_reduce_all(t, mean, &v1, &v2)) {
+            pg_node *n1 = reduce_attach(a, 0, false, false, v1);
+            if (!n1) {
+                pg_tensor_free(v2);
+                return NULL;
+            }
+            pg_node *out = reduce_attach(n1, 0, false, mean, v2);
+            pg_node_free(n1);
+            return out;
+        }
     }
     if (t->ndim == 2 && pgk_sum_all2s_fits(t->shape[0], t->shape[1])) {
         /* sliced column sums: the same sums in the same order as the

@@ -137,8 +137,8 @@ bool pgc_load_into(pg_tensor *dst, FILE *fp);
  * else is queued or waited on */
 bool pga_lazy_pending(void);
 void pga_lazy_flush(void);
-/* the pending small run and the fused backward region bwd in one launch
- * (true), or nothing launched (false) */
+/* the pending run and the fused backward region bwd in one launch (true),
+ * or nothing launched (false) */
 bool pga_lazy_flush_with_backward(const pg_jit_graph *bwd, size_t lnd, const size_t *ls, const void *const *bin,
                                   size_t bnin, void *const *bout, size_t bnout);
 /* t is the output of a pending op: the run is flushed with t's 16-bit copy
@@ -216,8 +216,11 @@ void pgj_mark_output16(pg_jit_graph *g, int id, int dt16);
 void pgj_graph_set_launder(pg_jit_graph *g);
 int pgj_op_internal(pg_jit_graph *g, int op, int a, int b);
 /* dst gains src's nodes (src input i -> dst node in_map[i]) and, after its
- * own, src's outputs, each of which must have the loop shape (lnd, ls) */
-bool pgj_graph_append(pg_jit_graph *dst, const pg_jit_graph *src, const int *in_map, size_t lnd, const size_t *ls);
+ * own, src's outputs; full: each must have the loop shape (lnd, ls), else
+ * src's nodes stay compiled as in src alone (contracted beside an exact dst) */
+bool pgj_graph_append(pg_jit_graph *dst, const pg_jit_graph *src, const int *in_map, size_t lnd, const size_t *ls,
+                      bool full);
+size_t pgj_output_bytes(const pg_jit_graph *g, size_t o);
 bool pgj_input_shape(const pg_jit_graph *g, size_t i, size_t *ndim, const size_t **shape);
 enum { PGJ_OP_GELU_GRAD = 100, PGJ_OP_SIGN = 101, PGJ_OP_ERF_GRAD = 102 };
 /* compile (cached) and launch with device pointers; loop shape given

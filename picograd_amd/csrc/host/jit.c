@@ -67,6 +67,7 @@ struct pg_jit_graph {
     jout outs[MAXIO * 2];
     size_t nout;
     bool exact; /* no FMA contraction between the graph's ops (pgj_graph_set_exact) */
+    size_t nexact; /* not exact as a whole: its first nexact nodes are (pgj_graph_append) */
     bool launder; /* stored values through one asm copy (pgj_graph_set_launder) */
 };
 
@@ -368,17 +369,23 @@ void pgj_mark_output16(pg_jit_graph *g, int id, int dt16)
 
 /* Appends src's nodes to dst: src's input i becomes dst's node in_map[i],
  * constants and ops are copied in order, and src's outputs are marked on
- * dst after dst's own (same shapes and betas).  Every output of src must be
- * a full loop-shape output (lnd, ls): the caller's one-block run stores
- * them element by element.  False when that fails (dst may hold unused
- * extra nodes then, and no extra outputs). */
-bool pgj_graph_append(pg_jit_graph *dst, const pg_jit_graph *src, const int *in_map, size_t lnd, const size_t *ls)
+ * dst after dst's own (same shapes and betas).  With full, every output of
+ * src must be a full loop-shape output (lnd, ls): the caller's one-block run
+ * stores them element by element.  Without it, an exact dst keeps its own
+ * nodes uncontracted and src's are compiled as in src alone.  False when
+ * that fails (dst may hold unused extra nodes then, and no extra outputs). */
+bool pgj_graph_append(pg_jit_graph *dst, const pg_jit_graph *src, const int *in_map, size_t lnd, const size_t *ls,
+                      bool full)
 {
     if (!dst || !src || dst->nout + src->nout > MAXIO * 2)
         return false;
-    for (size_t o = 0; o < src->nout; o++)
+    for (size_t o = 0; o < src->nout && full; o++)
         if (!pg_shape_equal(src->outs[o].ndim, src->outs[o].shape, lnd, ls))
             return false;
+    if (!full && dst->exact && !src->exact) {
+        dst->exact = false;
+        dst->nexact = dst->nn;
+    }
     int *map = malloc((src->nn ? src->nn : 1) * sizeof(int));
     if (!map)
         return false;
@@ -406,6 +413,14 @@ bool pgj_graph_append(pg_jit_graph *dst, const pg_jit_graph *src, const int *in_
     }
     free(map);
     return ok;
+}
+
+/* bytes of output o */
+size_t pgj_output_bytes(const pg_jit_graph *g, size_t o)
+{
+    if (!g || o >= g->nout)
+        return 0;
+    return pg_shape_numel(g->outs[o].ndim, g->outs[o].shape) * (g->outs[o].dt16 ? 2 : 4);
 }
 
 /* input i's shape */
@@ -456,6 +471,8 @@ uint64_t pg_jit_graph_hash(const pg_jit_graph *g)
     h = fnv(&g->nout, sizeof g->nout, h);
     if (g->exact)
         h = fnv("exact", 5, h);
+    if (g->nexact)
+        h = fnv(&g->nexact, sizeof g->nexact, h);
     if (g->launder)
         h = fnv("launder", 7, h);
     for (size_t i = 0; i < g->nout; i++)
@@ -487,7 +504,8 @@ uint64_t pg_jit_graph_hash(const pg_jit_graph *g)
 
 static bool graph_equal(const pg_jit_graph *a, const pg_jit_graph *b)
 {
-    if (a->nn != b->nn || a->nin != b->nin || a->nout != b->nout || a->exact != b->exact || a->launder != b->launder)
+    if (a->nn != b->nn || a->nin != b->nin || a->nout != b->nout || a->exact != b->exact || a->nexact != b->nexact ||
+        a->launder != b->launder)
         return false;
     for (size_t i = 0; i < a->nn; i++) {
         const jnode *x = &a->nodes[i], *y = &b->nodes[i];
@@ -546,6 +564,11 @@ typedef struct {
     int ksplit;
     int64_t R, C;
     int vec;
+    /* the [R x C] tiling: inputs that every row reads alike (loaded once per
+     * lane, before its rows; with four columns per lane that only costs registers), and streaming accesses kept to rows of whole
+     * 128-byte lines */
+    bool in_rowless[MAXIO * 2];
+    bool stream;
 } plan_t;
 
 /* strides (in elements) of a contiguous `shape` broadcast over the loop
@@ -728,6 +751,12 @@ static bool make_plan(const pg_jit_graph *g, size_t lnd, const size_t *ls, plan_
         if (P->in_used[i] && !(P->istr[i][nd - 1] == 0 || P->istr[i][nd - 1] == 1))
             v4 = false;
     P->vec = v4 ? 4 : 1;
+    P->stream = !any_red || P->C % 32 == 0;
+    for (int i = 0; i < P->nin && any_red; i++) {
+        P->in_rowless[i] = P->ksplit == nd - 1 && P->vec == 1;
+        for (int d = 0; d < P->ksplit; d++)
+            P->in_rowless[i] = P->in_rowless[i] && P->istr[i][d] == 0;
+    }
     return true;
 }
 
@@ -817,18 +846,24 @@ static void emit_loads(sbuf *b, const plan_t *P, int vec, const char *idx, int u
         if (!P->in_used[i])
             continue;
         int nid = P->in_node[i];
+        if (P->R > 0 && P->in_rowless[i]) { /* emit_rowless loaded it */
+            for (int e = 0; e < vec; e++)
+                sb_add(b, "    const float v%d_%d_%d = h%d_%d;\n", nid, u, e, nid, e);
+            continue;
+        }
         if (vec == 4 && P->istr[i][P->ndim - 1] != 0) {
             /* an input of the full loop shape is read exactly once: stream it
              * past the caches; broadcast inputs are re-read and stay cached */
-            if (P->in_direct[i])
+            const bool nt = P->in_direct[i] && P->stream;
+            if (nt)
                 sb_add(b, "    const pgf4 q%d_%d = __builtin_nontemporal_load((const pgf4 *)(in%d + ", nid, u, i);
             else
                 sb_add(b, "    const pgf4 q%d_%d = *(const pgf4 *)(in%d + ", nid, u, i);
             emit_offset(b, P, i, idx);
-            sb_add(b, P->in_direct[i] ? "));\n" : ");\n");
+            sb_add(b, nt ? "));\n" : ");\n");
             sb_add(b, "    float v%d_%d_0 = q%d_%d.x, v%d_%d_1 = q%d_%d.y, v%d_%d_2 = q%d_%d.z, v%d_%d_3 = q%d_%d.w;\n",
                    nid, u, nid, u, nid, u, nid, u, nid, u, nid, u, nid, u, nid, u);
-        } else if (P->in_direct[i]) {
+        } else if (P->in_direct[i] && P->stream) {
             sb_add(b, "    const float s%d_%d = __builtin_nontemporal_load(in%d + ", nid, u, i);
             emit_offset(b, P, i, idx);
             sb_add(b, ");\n");
@@ -840,6 +875,18 @@ static void emit_loads(sbuf *b, const plan_t *P, int vec, const char *idx, int u
         if (!(vec == 4 && P->istr[i][P->ndim - 1] != 0))
             for (int e = 0; e < vec; e++)
                 sb_add(b, "    float v%d_%d_%d = s%d_%d;\n", nid, u, e, nid, u);
+    }
+}
+
+/* the tiling's row-invariant inputs (a bias), once per lane at column c */
+static void emit_rowless(sbuf *b, const plan_t *P, int vec)
+{
+    for (int i = 0; i < P->nin; i++) {
+        if (!P->in_used[i] || !P->in_rowless[i])
+            continue;
+        for (int e = 0; e < vec; e++)
+            sb_add(b, "  const float h%d_%d = in%d[(c + %du) * (IDX)%lld];\n", P->in_node[i], e, i, e,
+                   (long long)P->istr[i][P->ndim - 1]);
     }
 }
 
@@ -867,9 +914,11 @@ static void emit_compute(sbuf *b, const pg_jit_graph *g, const bool *reach, int 
             char sa[40], sc[40];
             snprintf(sa, sizeof sa, "v%d_%d_%d", n->in[0], u, e);
             snprintf(sc, sizeof sc, "v%d_%d_%d", n->nin == 2 ? n->in[1] : n->in[0], u, e);
-            sb_add(b, "    const float v%zu_%d_%d = ", id, u, e);
+            /* an exact node beside contracted ones: off for its expression */
+            const bool off = !g->exact && id < g->nexact;
+            sb_add(b, "    const float v%zu_%d_%d = %s", id, u, e, off ? "({ _Pragma(\"clang fp contract(off)\") " : "");
             emit_expr(b, n, sa, sc);
-            sb_add(b, ";\n");
+            sb_add(b, off ? "; });\n" : ";\n");
         }
     }
 }
@@ -937,7 +986,18 @@ static void emit_stores(sbuf *b, const plan_t *P, int vec, const char *idx, int 
             continue;
         }
         /* each output element is written once per launch: stream the stores
-         * (and the read of an accumulating output) past the caches */
+         * (and the read of an accumulating output) past the caches.  Rows
+         * that end inside a 128-byte line keep ordinary ones: two waves write
+         * each such line, and only the caches can put it together */
+        if (!P->stream) {
+            const char *eq = P->out_beta[o] ? "+=" : "=";
+            if (vec == 4)
+                sb_add(b, "    *(pgf4 *)(out%d + %s) %s (pgf4){w%d_%d_0, w%d_%d_1, w%d_%d_2, w%d_%d_3};\n", o, idx, eq, nid, u,
+                       nid, u, nid, u, nid, u);
+            else
+                sb_add(b, "    out%d[%s] %s w%d_%d_0;\n", o, idx, eq, nid, u);
+            continue;
+        }
         if (vec == 4) {
             if (P->out_beta[o])
                 sb_add(b, "    { pgf4 *p = (pgf4 *)(out%d + %s); pgf4 t = __builtin_nontemporal_load(p);"
@@ -986,6 +1046,17 @@ static void emit_headers(sbuf *b, const plan_t *P)
         sb_add(b, "%s\ntypedef unsigned int pgu2 __attribute__((ext_vector_type(2)));\n", pgk_convert_source);
 }
 
+/* the [R x C] tiling's column lanes of 256: 64, or for few columns the power
+ * of two that covers them, so the other lanes take more rows instead of
+ * idling; the rest are row lanes */
+static int red_lanes(const plan_t *P, int vec)
+{
+    int n = 4;
+    while (n < 64 && (int64_t)n * vec < P->C)
+        n *= 2;
+    return n;
+}
+
 static char *gen_source(const pg_jit_graph *g, const plan_t *P, const bool *reach)
 {
     sbuf b = {0};
@@ -1030,33 +1101,51 @@ static char *gen_source(const pg_jit_graph *g, const plan_t *P, const bool *reac
         sb_add(&b, "  }\n}\n");
         return b.s;
     }
-    /* reduced outputs: [R x C] tiling; 64 column groups x 4 row lanes, each
-     * lane walking rows r, r+4, ... of its block's band, two per iteration */
+    /* reduced outputs: [R x C] tiling; 64 column groups x 4 row lanes (fewer
+     * x more for few columns), each lane walking rows r, r+4, ... of its
+     * block's band */
     int vec = (P->C % 4 == 0 && P->vec == 4) ? 4 : 1;
+    const int TC = red_lanes(P, vec), TR = 256 / TC;
     sb_add(&b, "extern \"C\" __global__ void __launch_bounds__(256) pgjit_main(PgArgs a) {\n");
     if (g->exact)
         sb_add(&b, "#pragma clang fp contract(off)\n");
     emit_prologue(&b, P);
     sb_add(&b, "  const IDX R = (IDX)%lldULL, C = (IDX)%lldULL;\n", (long long)P->R, (long long)P->C);
-    sb_add(&b, "  const IDX tc = threadIdx.x & 63u, tr = threadIdx.x >> 6;\n");
-    sb_add(&b, "  const IDX c = ((IDX)blockIdx.x * 64u + tc) * %du;\n", vec);
+    sb_add(&b, "  const IDX tc = threadIdx.x & %du, tr = threadIdx.x / %du;\n", TC - 1, TC);
+    sb_add(&b, "  unsigned bx = blockIdx.x, by = blockIdx.y;\n");
+    if (!P->stream) {
+        /* blocks side by side in a row share its unaligned lines: ids are
+         * dealt to the 8 XCDs round-robin, so they are regrouped to put
+         * neighbours on one XCD, whose L2 then holds the whole line */
+        sb_add(&b, "  {\n    const unsigned nb = gridDim.x * gridDim.y, id = by * gridDim.x + bx, q = nb >> 3;\n"
+                   "    const unsigned s = id < (q << 3) ? (id & 7u) * q + (id >> 3) : id;\n"
+                   "    by = s / gridDim.x; bx = s - by * gridDim.x;\n  }\n");
+    }
+    sb_add(&b, "  const IDX c = ((IDX)bx * %du + tc) * %du;\n", TC, vec);
     sb_add(&b, "  const IDX rows_per = (R + gridDim.y - 1) / gridDim.y;\n");
-    sb_add(&b, "  const IDX r0 = (IDX)blockIdx.y * rows_per;\n");
+    sb_add(&b, "  const IDX r0 = (IDX)by * rows_per;\n");
     sb_add(&b, "  const IDX r1 = r0 + rows_per < R ? r0 + rows_per : R;\n");
     for (int o = 0; o < P->nout; o++)
         if (P->out_red[o])
             for (int e = 0; e < vec; e++)
                 sb_add(&b, "  float acc%d_%d = 0.0f;\n", o, e);
     sb_add(&b, "  if (c < C) {\n");
+    emit_rowless(&b, P, vec);
     sb_add(&b, "  IDX r = r0 + tr;\n");
     /* PGJ_RED_ROWS rows per lane per iteration, all their loads issued
      * before the first compute; the column sums still add rows in order */
-    const int RU = PGJ_RED_ROWS;
+    int stored = 0;
+    for (int o = 0; o < P->nout; o++)
+        stored += !P->out_red[o];
+    /* fewer when many outputs are stored: their values hold registers, and a
+     * forward run with its backward (six stored arrays of [16384, 4096])
+     * takes 424 us with two rows, 440 with four */
+    const int RU = vec == 4 && stored > 4 ? PGJ_RED_ROWS / 2 : PGJ_RED_ROWS;
     static const char *const iname[8] = {"i0", "i1", "i2", "i3", "i4", "i5", "i6", "i7"};
-    sb_add(&b, "  for (; r + %du < r1; r += %du) {\n", 4 * (RU - 1), 4 * RU);
+    sb_add(&b, "  for (; r + %du < r1; r += %du) {\n", TR * (RU - 1), TR * RU);
     sb_add(&b, "    const IDX i0 = r * C + c");
     for (int u = 1; u < RU; u++)
-        sb_add(&b, ", i%d = i0 + %du * C", u, 4 * u);
+        sb_add(&b, ", i%d = i0 + %du * C", u, TR * u);
     sb_add(&b, ";\n");
     for (int u = 0; u < RU; u++)
         emit_loads(&b, P, vec, iname[u], u);
@@ -1072,7 +1161,7 @@ static char *gen_source(const pg_jit_graph *g, const plan_t *P, const bool *reac
                            P->out_node[o], u, e);
     for (int u = 0; u < RU; u++)
         emit_stores(&b, P, vec, iname[u], u);
-    sb_add(&b, "  }\n  for (; r < r1; r += 4u) {\n    const IDX i0 = r * C + c;\n");
+    sb_add(&b, "  }\n  for (; r < r1; r += %du) {\n    const IDX i0 = r * C + c;\n", TR);
     emit_loads(&b, P, vec, "i0", 0);
     emit_compute(&b, g, reach, vec, 0);
     emit_launder(&b, P, vec, 0);
@@ -1083,8 +1172,8 @@ static char *gen_source(const pg_jit_graph *g, const plan_t *P, const bool *reac
                        P->out_node[o], e);
     emit_stores(&b, P, vec, "i0", 0);
     sb_add(&b, "  }\n  }\n");
-    /* combine the 4 row lanes in LDS, fixed order, one partial row per block */
-    sb_add(&b, "  __shared__ float red[4][%d];\n", 64 * vec);
+    /* combine the row lanes in LDS, fixed order, one partial row per block */
+    sb_add(&b, "  __shared__ float red[%d][%d];\n", TR, TC * vec);
     for (int o = 0; o < P->nout; o++) {
         if (!P->out_red[o])
             continue;
@@ -1092,10 +1181,11 @@ static char *gen_source(const pg_jit_graph *g, const plan_t *P, const bool *reac
             sb_add(&b, "  red[tr][tc * %d + %d] = acc%d_%d;\n", vec, e, o, e);
         sb_add(&b, "  __syncthreads();\n");
         sb_add(&b, "  if (tr == 0 && c < C) {\n");
-        for (int e = 0; e < vec; e++)
-            sb_add(&b, "    a.part[%d][(IDX)blockIdx.y * C + c + %d] = ((red[0][tc*%d+%d] + red[1][tc*%d+%d]) + "
-                       "red[2][tc*%d+%d]) + red[3][tc*%d+%d];\n",
-                   o, e, vec, e, vec, e, vec, e, vec, e);
+        for (int e = 0; e < vec; e++) {
+            sb_add(&b, "    { float s = red[0][tc*%d+%d];\n", vec, e);
+            sb_add(&b, "#pragma unroll\n      for (int q = 1; q < %d; ++q) s += red[q][tc*%d+%d];\n", TR, vec, e);
+            sb_add(&b, "      a.part[%d][(IDX)by * C + c + %d] = s; }\n", o, e);
+        }
         sb_add(&b, "  }\n  __syncthreads();\n");
     }
     sb_add(&b, "}\n");
@@ -1439,8 +1529,9 @@ static centry *get_entry(const pg_jit_graph *g, size_t lnd, const size_t *ls, in
         e->grid_y = 1;
     } else {
         int vec = (P.C % 4 == 0 && P.vec == 4) ? 4 : 1;
-        int64_t cb = (P.C + 64 * vec - 1) / (64 * vec);
-        /* ~16K short-lived blocks of >= 16 rows (4 per row lane, one
+        const int tc = red_lanes(&P, vec), tr = 256 / tc;
+        int64_t cb = (P.C + tc * vec - 1) / (tc * vec);
+        /* ~16K short-lived blocks of >= 16 rows of wide outputs (4 per row lane, one
          * iteration of PGJ_RED_ROWS = 4): measured on the config-2 shape,
          * 16-row bands take 176 us with 2 rows per lane per iteration and
          * 173 us with 4, against 195 us for 32-row bands and 202 us for
@@ -1448,7 +1539,7 @@ static centry *get_entry(const pg_jit_graph *g, size_t lnd, const size_t *ls, in
         int64_t rb = 16384 / (cb ? cb : 1);
         if (rb < 1)
             rb = 1;
-        int64_t max_rb = (P.R + 15) / 16;
+        int64_t max_rb = (P.R + 4 * tr - 1) / (4 * tr);
         if (rb > max_rb)
             rb = max_rb;
         if (rb < 1)

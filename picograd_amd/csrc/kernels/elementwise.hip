@@ -336,6 +336,40 @@ __global__ void __launch_bounds__(kBlock) k_sum_axis_fin(const float *__restrict
     }
 }
 
+// y[0] = scale * sum of x[0 .. n), n of a few thousand: one block, each lane
+// adding x[t], x[t + 1024], ... in that order (four loads in flight), the
+// lanes by a fixed pairwise tree: one launch for the total of a wide
+// reduction's column sums, where k_sum_axis_part + _fin take two.
+constexpr int kSumVecThreads = 1024;
+__global__ void __launch_bounds__(kSumVecThreads) k_sum_vec(const float *__restrict__ x, float *__restrict__ y, int n,
+                                                            float scale)
+{
+    __shared__ float red[kSumVecThreads];
+    const int t = threadIdx.x;
+    float acc = 0.0f;
+    int i = t;
+    for (; i + 3 * kSumVecThreads < n; i += 4 * kSumVecThreads) {
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            v[q] = x[i + q * kSumVecThreads];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            acc += v[q];
+    }
+    for (; i < n; i += kSumVecThreads)
+        acc += x[i];
+    red[t] = acc;
+    __syncthreads();
+    for (int h = kSumVecThreads / 2; h > 0; h >>= 1) {
+        if (t < h)
+            red[t] += red[t + h];
+        __syncthreads();
+    }
+    if (t == 0)
+        y[0] = red[0] * scale;
+}
+
 // Both reductions of a [rows, cols] reduce_all in one block, when each is a
 // single run (sum_axis_plan gives one slice for both): lane j adds column j
 // over the rows in row order (y1[j], as k_sum_axis_part with one slice),
@@ -1318,6 +1352,14 @@ extern "C" int pgk_sum_axis_f32(const float *x, float *y, size_t outer, size_t l
     if (slices > 1)
         hipLaunchKernelGGL(k_sum_axis_fin, dim3(grid_for(n)), dim3(kBlock), 0, (hipStream_t)s, part, y, n, slices,
                            scale);
+    return status();
+}
+
+extern "C" int pgk_sum_vec_f32(const float *x, float *y, size_t n, float scale, pgk_stream s)
+{
+    if (!n || n > 0x7fffffff)
+        return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_sum_vec, dim3(1), dim3(kSumVecThreads), 0, (hipStream_t)s, x, y, (int)n, scale);
     return status();
 }
 

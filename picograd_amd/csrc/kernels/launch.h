@@ -86,6 +86,8 @@ int pgk_expand_into_f32(float *dst, const float *src, const pgk_bcast *bc, float
 size_t pgk_sum_axis_workspace(size_t outer, size_t len, size_t inner);
 int pgk_sum_axis_f32(const float *x, float *y, size_t outer, size_t len, size_t inner,
                      float scale, void *ws, pgk_stream s);
+/* y[0] = scale * (x[0] + ... + x[n - 1]) from one block, in a fixed order */
+int pgk_sum_vec_f32(const float *x, float *y, size_t n, float scale, pgk_stream s);
 /* Both stages of reduce_all over a contiguous [rows, cols] in one launch:
  * y1[cols] = column sums, y2[0] = scale * sum(y1), with the additions of
  * two pgk_sum_axis_f32 calls in their order.  Only where each stage is a
