@@ -145,8 +145,8 @@ size_t pg_amd_jit_cache_hits(void);
  * measurement and test aid): returns the tile (1: 128 x 128, four waves;
  * 2: 256 x 256, eight waves; 3: 128 x 256, eight waves; 4: the skinny
  * kernel for n <= 16 with B MN-contiguous and at least 1009 rows, 16 rows
- * of C per block, one launch with no split; 5, 6 and 7: tiles of 32 x 32,
- * 32 x 64 and 64 x 64 whose waves split the reduction, for outputs that
+ * of C per block, one launch with no split; 5 to 8: tiles of 32 x 32,
+ * 32 x 64 and 64 x 64 (two forms) whose waves split the reduction, for outputs that
  * 128-tiles would not spread over the chip), stores the
  * split-K factor (1 = none) in *splits and the planner's time estimate in
  * seconds in *seconds (either may be NULL).  cu_budget: the CUs the launch

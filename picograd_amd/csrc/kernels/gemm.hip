@@ -1171,13 +1171,13 @@ int launch_tile(const gemm_args &g, const pgk_epi &epi, hipStream_t s)
 }
 
 // the split-over-waves tiles of the planner: 5 is 32 x 32 with eight waves, 6
-// 32 x 64 with eight, 7 64 x 64 with four (two blocks per CU).  Deeper rings
-// and 64 x 64 with eight waves measured slower.
+// 32 x 64 with eight, 7 64 x 64 with four (two blocks per CU), 8 64 x 64 with
+// eight.  Deeper rings measured slower.
 template <int TILE, bool TA, bool TB, bool F16>
 using ks_cfg = typename std::conditional<
     TILE == 5, kscfg<32, 32, 8, 64, 2, TA, TB, F16>,
     typename std::conditional<TILE == 6, kscfg<32, 64, 8, 32, 3, TA, TB, F16>,
-                              kscfg<64, 64, 4, 32, 2, TA, TB, F16>>::type>::type;
+                              kscfg<64, 64, TILE == 8 ? 8 : 4, 32, 2, TA, TB, F16>>::type>::type;
 
 template <class CF>
 gemm_kargs ks_kargs(const gemm_args &g, const pgk_epi &epi)
@@ -1200,6 +1200,7 @@ int launch_ks_tile(const gemm_args &g, const pgk_epi &epi, int has_epi, hipStrea
     switch (g.tile) {
     case 5: return launch_ks<ks_cfg<5, TA, TB, F16>>(g, epi, has_epi, s);
     case 6: return launch_ks<ks_cfg<6, TA, TB, F16>>(g, epi, has_epi, s);
+    case 8: return launch_ks<ks_cfg<8, TA, TB, F16>>(g, epi, has_epi, s);
     default: return launch_ks<ks_cfg<7, TA, TB, F16>>(g, epi, has_epi, s);
     }
 }
@@ -1237,6 +1238,7 @@ int launch_ks_pair_tile(int tile, const gemm_args &gd, const gemm_args &gw, hipS
     switch (tile) {
     case 5: return launch_ks_pair<F16, 5>(gd, gw, s);
     case 6: return launch_ks_pair<F16, 6>(gd, gw, s);
+    case 8: return launch_ks_pair<F16, 8>(gd, gw, s);
     default: return launch_ks_pair<F16, 7>(gd, gw, s);
     }
 }
@@ -1413,7 +1415,7 @@ __global__ void __launch_bounds__(512, 1) k_mfma_probe(float *sink, int iters, i
 // Ragged shapes such as M = 4097 (33 rows of 128-tiles) and weight grads
 // with a short output dim are where it matters.
 typedef struct {
-    int tile; // 2 = 256 x 256, 3 = 128 x 256, 1 = 128 x 128, 5 - 7: ks_tile
+    int tile; // 2 = 256 x 256, 3 = 128 x 256, 1 = 128 x 128, 5 - 8: ks_tile
     int sp;   // split-K factor, 1 = none
 } gemm_plan;
 
@@ -1427,10 +1429,14 @@ static constexpr int kCUs = 256;
 // that count at every reduction measured (128 to 4096: 32 x 32 at 256 blocks
 // 3.7 - 13 against 7.2 - 20 us; 64 x 64 at 512 blocks 7.1 - 33 against 7.5 -
 // 36 us); past it they lose (64 x 64 at 1024 blocks 12 - 21 against 7.6 - 17
-// us).  Products of at most 16 columns keep their plans: more than half of
+// us).  A 64 x 64 tile takes eight waves in place of four for a long
+// reduction that leaves one block per CU: the same time (8.4 and 8.5 us at
+// 1024^3), and as many partial sums as the split-K plan there has, so the
+// error against 64 bits stays where it was (1.5e-7 at k = 4096, 1.9e-7 with
+// four).  Products of at most 16 columns keep their plans: more than half of
 // these tiles would be padding.
 struct ks_size {
-    size_t m, n, batch;
+    size_t m, n, batch, k;
 };
 static int ks_tile(std::initializer_list<ks_size> problems)
 {
@@ -1439,11 +1445,13 @@ static int ks_tile(std::initializer_list<ks_size> problems)
         size_t tm, tn, most;
     } shapes[3] = {{5, 32, 32, 256}, {6, 32, 64, 256}, {7, 64, 64, 512}};
     for (const auto &sh : shapes) {
-        size_t blocks = 0;
-        for (const ks_size &q : problems)
+        size_t blocks = 0, k = 0;
+        for (const ks_size &q : problems) {
             blocks += ((q.m + sh.tm - 1) / sh.tm) * ((q.n + sh.tn - 1) / sh.tn) * q.batch;
+            k = q.k > k ? q.k : k;
+        }
         if (blocks <= sh.most)
-            return sh.tile;
+            return sh.tile == 7 && blocks <= 256 && k >= 1024 ? 8 : sh.tile;
     }
     return 0;
 }
@@ -1470,7 +1478,7 @@ static gemm_plan plan_gemm(size_t m, size_t n, size_t kin, size_t batch, int cu_
 {
     const bool whole = !(cu_budget > 0 && cu_budget < kCUs);
     const double cus = whole ? (double)kCUs : (double)cu_budget;
-    const int ks = whole && n > 16 && kin ? ks_tile({{m, n, batch}}) : 0;
+    const int ks = whole && n > 16 && kin ? ks_tile({{m, n, batch, kin}}) : 0;
     if (ks) {
         if (time)
             *time = ks_time(ks, m, n, kin, batch);
@@ -1790,7 +1798,7 @@ extern "C" int pgk_gemm16_ks_pair_tile(const pgk_gemm_desc *d, const pgk_gemm_de
     if (!d->m || !d->n || !d->k || !d->batch || !w->m || !w->n || !w->k || !w->batch || d->k % 8 ||
         skinny_ok(1, 1, w->m, w->n, w->k, w->batch))
         return 0;
-    return ks_tile({{d->m, d->n, d->batch}, {w->m, w->n, w->batch}});
+    return ks_tile({{d->m, d->n, d->batch, d->k}, {w->m, w->n, w->batch, w->k}});
 }
 
 extern "C" int pgk_gemm16_ks_pair(int dtype, const pgk_gemm_desc *d, const pgk_gemm_desc *w, pgk_stream s)

@@ -193,7 +193,7 @@ typedef struct {
  * different tile sizes.  ws: pgk_gemm16_pair_dw_workspace bytes. */
 #define PGK_GEMM_NOT_PAIRED (-1)
 /* The same pair in one launch on a split-over-waves tile (pgk_gemm16_plan's
- * 5 to 7), no workspace; _tile is that tile, 0 when none holds both (the
+ * 5 to 8), no workspace; _tile is that tile, 0 when none holds both (the
  * launch is then refused as PGK_GEMM_NOT_PAIRED). */
 int pgk_gemm16_ks_pair_tile(const pgk_gemm_desc *d, const pgk_gemm_desc *w);
 int pgk_gemm16_ks_pair(int dtype, const pgk_gemm_desc *d, const pgk_gemm_desc *w, pgk_stream s);

@@ -1,5 +1,5 @@
-"""The 16-bit GEMM tiles whose waves split the reduction (planner tiles 5, 6
-and 7), at the sizes where they can go wrong: one element, tile edges, a
+"""The 16-bit GEMM tiles whose waves split the reduction (planner tiles 5 to
+8), at the sizes where they can go wrong: one element, tile edges, a
 reduction shorter than one wave's chunk, shorter than the eight waves'
 chunks, ending mid-chunk, and the largest outputs each tile takes.
 
@@ -26,6 +26,7 @@ SHAPES = [
     (5, 1, 17, 8), (5, 31, 33, 24), (5, 33, 40, 64), (5, 64, 512, 513), (5, 256, 1024, 520), (5, 250, 1023, 40),
     (6, 512, 1024, 256), (6, 510, 1021, 264), (6, 1, 16384, 32), (6, 288, 1000, 8),
     (7, 1024, 1024, 72), (7, 1023, 2047, 136), (7, 2048, 1024, 16), (7, 600, 1000, 1000),
+    (8, 600, 1000, 1024), (8, 1024, 1023, 1100),
 ]
 
 
@@ -60,7 +61,7 @@ def test_split_over_waves(lib, oracle, k, shape, lay, dt):  # noqa: F811
 
 
 @pytest.mark.parametrize("dt", [BF16, F16])
-@pytest.mark.parametrize("shape", [(40, 72, 104), (257, 264, 520), (130, 512, 1024), (500, 1000, 520), (96, 208, 616)],
+@pytest.mark.parametrize("shape", [(40, 72, 104), (257, 264, 520), (130, 512, 1024), (1030, 264, 520), (500, 1000, 520), (96, 208, 616)],
                          ids=lambda s: "%dx%dx%d" % s)
 def test_pair_in_one_launch(lib, oracle, k, shape, dt):  # noqa: F811
     """dX = G.W^T and dW = X^T.G of C = X.W, X [M, K], W [K, N]; dW accumulates."""
@@ -83,7 +84,7 @@ def test_pair_in_one_launch(lib, oracle, k, shape, dt):  # noqa: F811
         cx, cw = d.put(bx), d.put(bw)
         dd = GemmDesc(M, K, N, pg, N, 0, M, pw, N, 0, K, cx + GUARD * ldx * 4, ldx, 0, 1, 0)
         dwd = GemmDesc(K, N, M, px, K, 0, K, pg, N, 0, N, cw + GUARD * ldw * 4, ldw, 0, 1, 1)
-        assert k.pgk_gemm16_ks_pair_tile(C.byref(dd), C.byref(dwd)) in (5, 6, 7)
+        assert k.pgk_gemm16_ks_pair_tile(C.byref(dd), C.byref(dwd)) in (5, 6, 7, 8)
         assert fn(dt, C.byref(dd), C.byref(dwd), k.pgd_stream()) == 0
         ax = d.get(cx, bx.shape, np.float32)
         aw = d.get(cw, bw.shape, np.float32)
