@@ -977,6 +977,128 @@ __global__ void __launch_bounds__(C1::NT, 1) k_gemm16_ks_pair(gemm_kargs g1, gem
         ks_block<C2>(g2, 0, (b - n1) % nb2, nb2, (n1 & 7) == 0, (b - n1) / nb2, (LDS uint4 *)smem);
 }
 
+// Few rows: C[m, n] (+)= A . B with A K-contiguous and B MN-contiguous, m <= 16
+// (a forward over a handful of inputs; up to 64 for at most 16 columns).  Such
+// a product streams B once, so a block owns 16 columns of one 16-row tile (256
+// blocks for 4096 columns: every CU streams) and its eight waves split the
+// reduction as k_gemm16_ks's do, each with a three-stage ring of 64-deep
+// chunks of its own.  Tiles of 16 x 16 (v_mfma_f32_16x16x32) halve what A costs
+// the 32-row ones.  Bound by the stream of 32-byte row pieces: 16 x 4096 x 4096
+// takes 11.7 us (2.9 TB/s; 64-column pieces would take 8.8 without the sum
+// across blocks that they need), against 14.3 on 32 x 32 tiles and 19 for
+// split-K and its sum; 16 x 10 x 4096 takes 4.6 us against 10.8.  Two or four
+// stages, sixteen waves and 32 columns a block measured the same or slower.
+typedef float f32x4m __attribute__((ext_vector_type(4)));
+
+template <bool F16>
+__device__ __forceinline__ f32x4m mfma16(const uint4 &a, const uint4 &b, const f32x4m &c)
+{
+    if constexpr (F16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
+                                                      0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                       0, 0, 0);
+}
+
+constexpr int kFrWaves = 8, kFrStages = 3, kFrTile = 16, kFrK = 64;
+constexpr int kFrA = kFrTile * kFrK / 8, kFrB = kFrK * kFrTile / 8; // uint4 of one A and one B stage
+
+template <bool F16>
+__global__ void __launch_bounds__(kFrWaves * 64, 1) k_few_rows(gemm_kargs g, int has_epi)
+{
+    __shared__ uint4 smem[kFrWaves * kFrStages * (kFrA + kFrB)];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // neighbouring column tiles share each 128-byte line of a row: on one XCD
+    int pid = (int)blockIdx.x;
+    const int nb = (int)gridDim.x;
+    if ((nb & 7) == 0)
+        pid = (pid & 7) * (nb >> 3) + (pid >> 3);
+    const int n0 = pid * kFrTile, m0 = (int)blockIdx.y * kFrTile;
+    LDS uint4 *const ring = (LDS uint4 *)smem + wave * kFrStages * (kFrA + kFrB);
+    using TK = TileK<kFrTile, 64, kFrK>;
+    static_assert(TK::NQ == 2 && kFrB == 128, "two loads of A and two of B per stage");
+    constexpr int LPT = 4;
+    const int nct = (g.K + kFrK - 1) / kFrK, nc = nct > wave ? (nct - wave + kFrWaves - 1) / kFrWaves : 0;
+    // this wave's chunk c (chunk c * waves + wave of the reduction) into stage
+    // st; k at or past K reads the zero page
+    auto load = [&](int c, int st) {
+        const int ch = c * kFrWaves + wave, k0 = ch < nct ? ch * kFrK : g.K;
+        LDS uint4 *sa = ring + st * (kFrA + kFrB), *sb = sa + kFrA;
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            TK::load_q(q, g.A, g.lda, m0, g.a_extent, k0, g.K, sa, lane);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) { // [64 k][16 columns]: two 16-byte chunks per k row
+            const int slot = q * 64 + lane, k = slot >> 1;
+            int col = n0 + (slot & 1) * 8;
+            col = col < g.b_extent ? col : g.b_extent - 8;
+            const void *src = k0 + k < g.K ? (const void *)(g.B + (size_t)(k0 + k) * g.ldb + col) : (const void *)&g_zero16;
+            dma16(src, sb + q * 64);
+        }
+    };
+    const int grp = lane >> 4, q16 = lane & 15;
+    f32x4m acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (nc > 0) {
+#pragma unroll
+        for (int s = 0; s < kFrStages; ++s)
+            load(s, s);
+        int st = 0;
+        for (int c = 0; c < nc; ++c) {
+            const LDS uint4 *sa = ring + st * (kFrA + kFrB), *sb = sa + kFrA;
+            // chunk c landed (the newest kFrStages - 1 chunks may be in flight)
+            __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm((kFrStages - 1) * LPT));
+            __asm__ volatile("" ::: "memory");
+            // 16-lane group grp holds k = 32 s + 8 grp .. + 7 of row (A) or
+            // column (B) lane % 16; B from two transposing reads
+            uint4 fa[2], fb[2];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const u32x4 v = ((const LDS u32x4 *)sa)[q16 * TK::CH + TK::swz(4 * s + grp, q16)];
+                fa[s] = __builtin_bit_cast(uint4, v);
+                uint2 h2[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int k = 32 * s + 8 * grp + 4 * h + (q16 >> 2);
+                    h2[h] = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                          (LDS v4s *)((const LDS char *)sb + k * 32 + (q16 & 3) * 8)));
+                }
+                fb[s] = make_uint4(h2[0].x, h2[0].y, h2[1].x, h2[1].y);
+            }
+            // the stage's reads are done before its refill
+            __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(63));
+            __asm__ volatile("" ::: "memory");
+            load(c + kFrStages, st);
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                acc = mfma16<F16>(fa[s], fb[s], acc);
+            st = st + 1 == kFrStages ? 0 : st + 1;
+        }
+        __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(0));
+    }
+    __syncthreads(); // the rings are done: the waves' partials through LDS, added in wave order
+    constexpr int RP = kFrTile + 1;
+    LDS float *part = (LDS float *)smem;
+    static_assert(kFrWaves * kFrTile * RP * 4 <= (int)sizeof(smem), "partials fit the rings");
+#pragma unroll
+    for (int e = 0; e < 4; ++e) // lane holds column lane % 16 of rows 4 (lane / 16) + e
+        part[(wave * kFrTile + 4 * grp + e) * RP + q16] = acc[e];
+    __syncthreads();
+    const int t = (int)threadIdx.x, row = t >> 4, col = t & 15;
+    if (row < kFrTile && m0 + row < g.M && n0 + col < g.N) {
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kFrWaves; ++w)
+            v += part[(w * kFrTile + row) * RP + col];
+        const size_t off = (size_t)(m0 + row) * g.ldc + n0 + col;
+        if (has_epi)
+            epi_store(g.epi, g.C, off, n0 + col, v);
+        else
+            g.C[off] = g.beta ? g.C[off] + v : v;
+    }
+}
+
 // the same epilogue as a pass over a finished C (k-tail runs)
 __global__ void __launch_bounds__(256) k_bias_act(float *__restrict__ c, size_t ldc, int m, int n, pgk_epi epi)
 {
@@ -1531,6 +1653,14 @@ static bool skinny_ok(int ta, int tb, size_t m, size_t n, size_t k, size_t batch
     return tb && n <= 16 && batch == 1 && k && (ta || k % 8 == 0) && (m + 15) / 16 >= 64;
 }
 
+// k_few_rows's products: one 16-row tile with a block per CU at most (past
+// 4096 columns the wider tiles stream faster: 22.5 against 37.5 us at 11008),
+// or a few such tiles of one column tile
+static bool few_rows_ok(int ta, int tb, size_t m, size_t n, size_t k, size_t batch)
+{
+    return !ta && tb && batch == 1 && k && k % 8 == 0 && ((m <= 16 && n <= 4096) || (m <= 64 && n <= 16));
+}
+
 static size_t tail_ws(int ta, int tb, size_t m, size_t n, size_t k, size_t batch)
 {
     if (k_inkernel(ta, tb, k) == k)
@@ -1561,7 +1691,7 @@ int check_gemm_args(int ta, int tb, size_t m, size_t n, size_t k, const uint16_t
 
 extern "C" size_t pgk_gemm16_workspace_cu(int ta, int tb, size_t m, size_t n, size_t k, size_t batch, int cu_budget)
 {
-    if (skinny_ok(ta, tb, m, n, k, batch))
+    if (skinny_ok(ta, tb, m, n, k, batch) || few_rows_ok(ta, tb, m, n, k, batch))
         return 0;
     const gemm_plan pl = plan_gemm(m, n, k_inkernel(ta, tb, k), batch, cu_budget);
     const size_t part = pl.sp > 1 ? (((size_t)pl.sp * m * n * sizeof(float) + 255) & ~(size_t)255) : 0;
@@ -1575,10 +1705,10 @@ extern "C" size_t pgk_gemm16_workspace(int ta, int tb, size_t m, size_t n, size_
 
 extern "C" int pgk_gemm16_plan(int ta, int tb, size_t m, size_t n, size_t k, size_t batch, int cu_budget, int *splits)
 {
-    if (skinny_ok(ta, tb, m, n, k, batch)) {
+    if (skinny_ok(ta, tb, m, n, k, batch) || few_rows_ok(ta, tb, m, n, k, batch)) {
         if (splits)
             *splits = 1;
-        return 4;
+        return skinny_ok(ta, tb, m, n, k, batch) ? 4 : 9;
     }
     const gemm_plan pl = plan_gemm(m, n, k_inkernel(ta, tb, k), batch, cu_budget);
     if (splits)
@@ -1590,6 +1720,8 @@ extern "C" double pgk_gemm16_time(int ta, int tb, size_t m, size_t n, size_t k, 
 {
     if (skinny_ok(ta, tb, m, n, k, batch)) // A streamed once at ~5 TB/s, one launch
         return (double)(m * k * 2 + k * 32 + m * n * 4) / 5.0e12 + 5e-6;
+    if (few_rows_ok(ta, tb, m, n, k, batch)) // B streamed once
+        return (double)(n * k * 2) / 3.7e12 + 3.5e-6;
     double t = 0.0;
     plan_gemm(m, n, k_inkernel(ta, tb, k), batch, cu_budget, &t);
     return t;
@@ -1653,6 +1785,16 @@ extern "C" int pgk_gemm16_cu(int dtype, int ta, int tb, size_t m, size_t n, size
                 hipLaunchKernelGGL((k_skinny<false, false>), grid, dim3(kSkWaves * 64), 0, st, a, lda, (int)a_extent, b, ldb,
                                    (int)b_extent, c, ldc, (int)m, (int)n, (int)k, beta, e, he);
         }
+        return (int)hipGetLastError();
+    }
+    if (few_rows_ok(ta, tb, m, n, k, batch)) {
+        gemm_args g = {a, lda, 0, (int)a_extent, b, ldb, 0, (int)b_extent, c, ldc, 0, (int)m, (int)n, (int)k, beta, 1u};
+        const gemm_kargs kg = make_kargs<gcfg<64, 64, 1, 1, false, true, false, false, 64, 2>>(g, has_epi ? *epi : pgk_epi{});
+        const dim3 grid((unsigned)((n + kFrTile - 1) / kFrTile), (unsigned)((m + kFrTile - 1) / kFrTile));
+        if (f16)
+            hipLaunchKernelGGL(k_few_rows<true>, grid, dim3(kFrWaves * 64), 0, st, kg, (int)has_epi);
+        else
+            hipLaunchKernelGGL(k_few_rows<false>, grid, dim3(kFrWaves * 64), 0, st, kg, (int)has_epi);
         return (int)hipGetLastError();
     }
     const gemm_plan pl = plan_gemm(m, n, kmain, batch, cu_budget);

@@ -23,8 +23,8 @@ pytestmark = pytest.mark.gpu
 
 # (tile, m, n, k)
 SHAPES = [
-    (5, 1, 17, 8), (5, 31, 33, 24), (5, 33, 40, 64), (5, 64, 512, 513), (5, 256, 1024, 520), (5, 250, 1023, 40),
-    (6, 512, 1024, 256), (6, 510, 1021, 264), (6, 1, 16384, 32), (6, 288, 1000, 8),
+    (5, 17, 17, 8), (5, 31, 33, 24), (5, 33, 40, 64), (5, 64, 512, 513), (5, 256, 1024, 520), (5, 250, 1023, 40),
+    (6, 512, 1024, 256), (6, 510, 1021, 264), (6, 17, 16384, 32), (6, 288, 1000, 8),
     (7, 1024, 1024, 72), (7, 1023, 2047, 136), (7, 2048, 1024, 16), (7, 600, 1000, 1000),
     (8, 600, 1000, 1024), (8, 1024, 1023, 1100),
 ]
@@ -51,6 +51,32 @@ def test_split_over_waves(lib, oracle, k, shape, lay, dt):  # noqa: F811
     try:
         pa, pb, pc = d.put(a_st), d.put(b_st), d.put(buf)
         rc = k.pgk_gemm16_cu(dt, ta, tb, m, n, kk, pa, lda, 0, a_ext, pb, ldb, 0, b_ext, pc + GUARD * ldc * 4, ldc,
+                             0, 1, beta, None, None, 0, k.pgd_stream())
+        assert rc == 0, rc
+        after = d.get(pc, buf.shape, np.float32)
+    finally:
+        d.free()
+    _check_guards(after, m, n, what)
+    check_product(after[GUARD:GUARD + m, :n], [(_f32(dt, A), _f32(dt, B))], what, add=c0)
+
+
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("beta", [0, 1])
+@pytest.mark.parametrize("m,n,kk", [(1, 1, 8), (1, 4096, 1024), (15, 17, 72), (16, 4095, 520), (5, 10, 4096), (64, 16, 584),
+                                    (49, 7, 64), (16, 128, 8192)])
+def test_few_rows(lib, oracle, k, m, n, kk, beta, dt):  # noqa: F811
+    what = f"few rows dt={dt} {m}x{n}x{kk} beta={beta}"
+    print(what, flush=True)
+    sp = C.c_int(0)
+    assert k.pgk_gemm16_plan(0, 1, m, n, kk, 1, 0, C.byref(sp)) == 9 and sp.value == 1
+    assert k.pgk_gemm16_workspace_cu(0, 1, m, n, kk, 1, 0) == 0
+    rng = np.random.default_rng(m * 31 + n * 7 + kk)
+    A, B, a_st, lda, a_ext, b_st, ldb, b_ext = _operands(oracle, rng, dt, 0, 1, m, n, kk)
+    buf, ldc, c0 = _c_buffer(rng, m, n, beta)
+    d = Dev(k)
+    try:
+        pa, pb, pc = d.put(a_st), d.put(b_st), d.put(buf)
+        rc = k.pgk_gemm16_cu(dt, 0, 1, m, n, kk, pa, lda, 0, a_ext, pb, ldb, 0, b_ext, pc + GUARD * ldc * 4, ldc,
                              0, 1, beta, None, None, 0, k.pgd_stream())
         assert rc == 0, rc
         after = d.get(pc, buf.shape, np.float32)
