@@ -194,19 +194,29 @@ struct F32Tile {
     }
 };
 
-template <int BM, int BN, int WGM, int WGN, int KB, bool TA, bool TB, bool VEC>
-__global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_f32(f32_args g)
+//
+// With KG = 2 the block has two groups of WGM x WGN waves: each computes the
+// whole tile over half of every k-tile, group 0 stages A and group 1 B, and
+// group 1's sums are added through LDS at the end.  Twice the waves per SIMD
+// for the same LDS, so one group's MFMAs cover the other's waits: for 256
+// blocks or fewer, one per CU, 1024 x 1024 x 2048 goes from 57 - 67 to 50 - 56
+// us; with two blocks per CU it measured the same, and slower on 128 x 128.
+template <int BM, int BN, int WGM, int WGN, int KB, int KG, bool TA, bool TB, bool VEC>
+__global__ void __launch_bounds__(64 * WGM * WGN * KG) k_gemm_f32(f32_args g)
 {
-    constexpr int NT = 64 * WGM * WGN, FM = BM / WGM / 32, FN = BN / WGN / 32, KS = KB / 8;
+    constexpr int NT = 64 * WGM * WGN, FM = BM / WGM / 32, FN = BN / WGN / 32, KS = KB / 8, KW = KS / KG;
     using OA = F32Tile<BM, KB, NT, TA, VEC>;
     using OB = F32Tile<BN, KB, NT, !TB, VEC>;
-    __shared__ f32x4 sa[2][OA::SLOTS], sb[2][OB::SLOTS];
+    __shared__ __align__(64) f32x4 smem[2 * (OA::SLOTS + OB::SLOTS)];
+    f32x4(*const sa)[OA::SLOTS] = (f32x4(*)[OA::SLOTS])smem;
+    f32x4(*const sb)[OB::SLOTS] = (f32x4(*)[OB::SLOTS])(smem + 2 * OA::SLOTS);
     const float *__restrict__ A = g.a + (size_t)blockIdx.z * g.sa;
     const float *__restrict__ B = g.b + (size_t)blockIdx.z * g.sb;
     float *__restrict__ C = g.c + (size_t)blockIdx.z * g.sc;
     const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
     const int m0 = tile / g.tiles_n * BM, n0 = tile % g.tiles_n * BN;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+    const int tid = threadIdx.x - grp * NT, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WGN * (BM / WGM), wn = wave % WGN * (BN / WGN);
     f32x16 acc[FM][FN];
 #pragma unroll
@@ -216,19 +226,27 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_f32(f32_args g)
 #pragma unroll
             for (int e = 0; e < 16; ++e)
                 acc[i][j][e] = 0.0f;
+    static_assert(KG == 1 || (KG == 2 && OA::NL == OB::NL && KS % 4 == 0), "one staging register set per group");
     OA ta;
     OB tb;
-    ta.init(g.lda, m0, g.m, tid);
-    tb.init(g.ldb, n0, g.n, tid);
-    f32x4 ra[OA::NL], rb[OB::NL];
+    if (KG == 1 || grp == 0)
+        ta.init(g.lda, m0, g.m, tid);
+    if (KG == 1 || grp == 1)
+        tb.init(g.ldb, n0, g.n, tid);
+    f32x4 ra[OA::NL], rb2[KG == 1 ? OB::NL : 1];
+    f32x4(&rb)[OB::NL] = *(f32x4(*)[OB::NL])(KG == 1 ? (void *)rb2 : (void *)ra);
     const int kt = g.k / KB + (g.k % KB != 0);
     auto store = [&](int buf) {
-        OA::store(ra, sa[buf], tid);
-        OB::store(rb, sb[buf], tid);
+        if (KG == 1 || grp == 0)
+            OA::store(ra, sa[buf], tid);
+        if (KG == 1 || grp == 1)
+            OB::store(rb, sb[buf], tid);
     };
     auto load = [&](int t) {
-        OA::load(ra, A, g.lda, m0, g.m, t * KB, g.k, tid);
-        OB::load(rb, B, g.ldb, n0, g.n, t * KB, g.k, tid);
+        if (KG == 1 || grp == 0)
+            OA::load(ra, A, g.lda, m0, g.m, t * KB, g.k, tid);
+        if (KG == 1 || grp == 1)
+            OB::load(rb, B, g.ldb, n0, g.n, t * KB, g.k, tid);
     };
     auto compute = [&](const f32x4 *ca, const f32x4 *cb, int s0, int s1) {
 #pragma unroll
@@ -236,10 +254,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_f32(f32_args g)
             f32x4 fa[FM], fb[FN];
 #pragma unroll
             for (int i = 0; i < FM; ++i)
-                fa[i] = OA::frag(ca, wm + 32 * i, s, lane);
+                fa[i] = OA::frag(ca, wm + 32 * i, grp * KW + s, lane);
 #pragma unroll
             for (int j = 0; j < FN; ++j)
-                fb[j] = OB::frag(cb, wn + 32 * j, s, lane);
+                fb[j] = OB::frag(cb, wn + 32 * j, grp * KW + s, lane);
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -259,20 +277,41 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_f32(f32_args g)
     const int fast = g.lda < ((size_t)1 << 22) && g.ldb < ((size_t)1 << 22) ? g.k / KB - 1 : 0;
     int t = 0;
     for (; t < fast; ++t) {
-        ta.load_fast(ra, A, g.lda, m0, (t + 1) * KB);
-        tb.load_fast(rb, B, g.ldb, n0, (t + 1) * KB);
-        compute(sa[t & 1], sb[t & 1], 0, KS * 3 / 4);
+        if (KG == 1 || grp == 0)
+            ta.load_fast(ra, A, g.lda, m0, (t + 1) * KB);
+        if (KG == 1 || grp == 1)
+            tb.load_fast(rb, B, g.ldb, n0, (t + 1) * KB);
+        compute(sa[t & 1], sb[t & 1], 0, KW * 3 / 4);
         store((t + 1) & 1);
-        compute(sa[t & 1], sb[t & 1], KS * 3 / 4, KS);
+        compute(sa[t & 1], sb[t & 1], KW * 3 / 4, KW);
         __syncthreads();
     }
     for (; t < kt; ++t) {
         if (t + 1 < kt)
             load(t + 1);
-        compute(sa[t & 1], sb[t & 1], 0, KS);
+        compute(sa[t & 1], sb[t & 1], 0, KW);
         if (t + 1 < kt)
             store((t + 1) & 1);
         __syncthreads();
+    }
+    if constexpr (KG == 2) { // after the last tile's barrier the buffers are free
+        f32x16 *part = (f32x16 *)smem;
+        static_assert(FM * FN * NT * 64 <= (int)sizeof smem, "group 1's sums fit");
+        if (grp) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+                    part[(i * FN + j) * NT + tid] = acc[i][j];
+        }
+        __syncthreads();
+        if (grp)
+            return;
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                acc[i][j] += part[(i * FN + j) * NT + tid];
     }
     // lane holds column lane % 32 of rows 8 (e / 4) + 4 (lane / 32) + e % 4
 #pragma unroll
@@ -383,27 +422,27 @@ __global__ void __launch_bounds__(64 * kSmWaves) k_gemm_f32_small(f32_args g)
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int KB, bool VEC>
+template <int BM, int BN, int WGM, int WGN, int KB, int KG, bool VEC>
 void launch_tiled_v(int ta, int tb, const f32_args &g, dim3 grid, hipStream_t s)
 {
-    const dim3 block(64 * WGM * WGN);
+    const dim3 block(64 * WGM * WGN * KG);
     switch ((ta ? 2 : 0) | (tb ? 1 : 0)) {
-    case 0: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, false, false, VEC>), grid, block, 0, s, g); break;
-    case 1: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, false, true, VEC>), grid, block, 0, s, g); break;
-    case 2: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, true, false, VEC>), grid, block, 0, s, g); break;
-    default: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, true, true, VEC>), grid, block, 0, s, g); break;
+    case 0: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, KG, false, false, VEC>), grid, block, 0, s, g); break;
+    case 1: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, KG, false, true, VEC>), grid, block, 0, s, g); break;
+    case 2: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, KG, true, false, VEC>), grid, block, 0, s, g); break;
+    default: hipLaunchKernelGGL((k_gemm_f32<BM, BN, WGM, WGN, KB, KG, true, true, VEC>), grid, block, 0, s, g); break;
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int KB>
+template <int BM, int BN, int WGM, int WGN, int KB, int KG = 1>
 void launch_tiled(int ta, int tb, f32_args g, unsigned batch, hipStream_t s)
 {
     g.tiles_n = (g.n + BN - 1) / BN;
     const dim3 grid((unsigned)((g.m + BM - 1) / BM) * (unsigned)g.tiles_n, 1, batch);
     if (g.va && g.vb)
-        launch_tiled_v<BM, BN, WGM, WGN, KB, true>(ta, tb, g, grid, s);
+        launch_tiled_v<BM, BN, WGM, WGN, KB, KG, true>(ta, tb, g, grid, s);
     else
-        launch_tiled_v<BM, BN, WGM, WGN, KB, false>(ta, tb, g, grid, s);
+        launch_tiled_v<BM, BN, WGM, WGN, KB, KG, false>(ta, tb, g, grid, s);
 }
 
 void launch_small(int ta, int tb, f32_args g, unsigned batch, hipStream_t s)
@@ -435,14 +474,17 @@ extern "C" int pgk_gemm_f32(int ta, int tb, size_t m, size_t n, size_t k, const 
     // 512 blocks and one of at most 256 (one per CU, which runs a block
     // faster but leaves the CU short of waves), in units of 39 us at k = 1024.
     // Measured there: 128 x 128 tiles 137 and 95 us, 64 x 64 tiles 39 and
-    // 33 us, 32 x 32 tiles with the reduction split over the waves 25 and 14 us
+    // 28 us (33 with one wave group), 32 x 32 tiles with the reduction split
+    // over the waves 25 and 14 us
     auto cost = [&](size_t tile, double full, double half) {
         const size_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * batch, rem = tiles % 512;
         return (double)(tiles / 512) * full + (rem > 256 ? full : rem ? half : 0.0);
     };
-    const double big = cost(128, 3.5, 2.4), mid = cost(64, 1.0, 0.85), small = cost(32, 0.64, 0.36);
+    const double big = cost(128, 3.5, 2.4), mid = cost(64, 1.0, 0.7), small = cost(32, 0.64, 0.36);
     if (small <= mid && small <= big)
         launch_small(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+    else if (mid <= big && ((m + 63) / 64) * ((n + 63) / 64) * batch <= 256)
+        launch_tiled<64, 64, 2, 2, 64, 2>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
     else if (mid <= big)
         launch_tiled<64, 64, 2, 2, 64>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
     else
