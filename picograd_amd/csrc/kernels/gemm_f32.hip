@@ -82,6 +82,11 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, const f32x16 &c)
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, const f32x4 &c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
 // Tiled kernel: a block of WGM x WGN waves owns BM x BN of C, each wave
 // (BM / WGM) x (BN / WGN) of it.  K-tiles of KB go global -> registers ->
 // LDS, the next tile's loads in flight while the current one is computed,
@@ -332,36 +337,39 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG) k_gemm_f32(f32_args g)
         }
 }
 
-// Small outputs: a block owns one 32 x 32 tile of C and its eight waves split
-// the reduction, each streaming its k range from global memory straight into
-// MFMA operands (no LDS, no barrier in the k-loop; 32 k in flight ahead of
-// the MFMAs).  The waves' partial tiles are added through LDS in wave order.
-// For outputs with too few 64 x 64 tiles for the chip, where one wave's serial
-// reduction would be the whole time: 256 x 784 x 512 takes 11 us, against
-// 24 - 28 us on 64 x 64 tiles and 103 us for the vector-FMA kernel before it.
+// Small outputs: a block owns one T x T tile of C (T = 16 or 32) and its eight
+// waves split the reduction, each streaming its k range from global memory
+// straight into MFMA operands (no LDS, no barrier in the k-loop; 1024 / T k in
+// flight ahead of the MFMAs).  The waves' partial tiles are added through LDS
+// in wave order.  For outputs with too few 64 x 64 tiles for the chip, where
+// one wave's serial reduction would be the whole time.  Bound by the chain of
+// load latencies along a wave's k range, which is why T = 16 is the faster one
+// while its blocks all run at once: 256 x 512 x 784 takes 7.9 - 8.8 us at
+// T = 16, 10.1 - 11.3 at T = 32 and 21 - 24 us on 64 x 64 tiles (103 us on the
+// vector-FMA kernel before them); 32 x 32 x 4096 12 - 17, 32 - 37 and 85 - 92.
 constexpr int kSmWaves = 8, kSmUnroll = 4;
 
-template <bool TA, bool TB>
-__global__ void __launch_bounds__(64 * kSmWaves) k_gemm_f32_small(f32_args g)
+template <int T, bool TA, bool TB>
+__device__ __forceinline__ void f32_small_block(const f32_args &g, const int tile, float (*part)[T][T + 1])
 {
-    __shared__ float part[kSmWaves][32][33];
+    constexpr int KS = 256 / T; // k per MFMA group: four from each T-lane part of the wave
+    typedef float acc_t __attribute__((ext_vector_type(T * T / 64)));
     const float *__restrict__ A = g.a + (size_t)blockIdx.z * g.sa;
     const float *__restrict__ B = g.b + (size_t)blockIdx.z * g.sb;
     float *__restrict__ C = g.c + (size_t)blockIdx.z * g.sc;
-    const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
-    const int m0 = tile / g.tiles_n * 32, n0 = tile % g.tiles_n * 32;
+    const int m0 = tile / g.tiles_n * T, n0 = tile % g.tiles_n * T;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // this wave's k range, whole groups of 8
-    const int kw = g.k ? (g.k - 1) / (8 * kSmWaves) * 8 + 8 : 0;
+    // this wave's k range, whole groups of KS
+    const int kw = g.k ? (g.k - 1) / (KS * kSmWaves) * KS + KS : 0;
     const int kb = wave * kw < g.k ? wave * kw : g.k;
     const int kend = g.k - kb > kw ? kb + kw : g.k;
-    const int row = m0 + (lane & 31) < g.m ? m0 + (lane & 31) : g.m - 1;
-    const int col = n0 + (lane & 31) < g.n ? n0 + (lane & 31) : g.n - 1;
-    const int kh = 4 * (lane >> 5);
-    f32x16 acc;
+    const int row = m0 + lane % T < g.m ? m0 + lane % T : g.m - 1;
+    const int col = n0 + lane % T < g.n ? n0 + lane % T : g.n - 1;
+    const int kh = 4 * (lane / T);
+    acc_t acc;
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
+    for (int e = 0; e < T * T / 64; ++e)
         acc[e] = 0.0f;
     auto mm = [&](const f32x4 &x, const f32x4 &y) {
 #pragma unroll
@@ -369,25 +377,25 @@ __global__ void __launch_bounds__(64 * kSmWaves) k_gemm_f32_small(f32_args g)
             acc = mfma_f32(x[q], y[q], acc);
     };
     constexpr int U = kSmUnroll;
-    const int whole = kb + (kend - kb) / (8 * U) * (8 * U);
+    const int whole = kb + (kend - kb) / (KS * U) * (KS * U);
     f32x4 fa[2][U], fb[2][U];
     auto load = [&](int buf, int k) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            fa[buf][u] = load_k4_full<TA>(A, g.lda, row, k + 8 * u + kh, g.va);
-            fb[buf][u] = load_k4_full<!TB>(B, g.ldb, col, k + 8 * u + kh, g.vb);
+            fa[buf][u] = load_k4_full<TA>(A, g.lda, row, k + KS * u + kh, g.va);
+            fb[buf][u] = load_k4_full<!TB>(B, g.ldb, col, k + KS * u + kh, g.vb);
         }
     };
     int k = kb;
     if (k < whole) {
         load(0, k);
-        for (; whole - k >= 16 * U; k += 16 * U) {
-            load(1, k + 8 * U);
+        for (; whole - k >= 2 * KS * U; k += 2 * KS * U) {
+            load(1, k + KS * U);
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 mm(fa[0][u], fb[0][u]);
-            if (whole - k > 16 * U)
-                load(0, k + 16 * U);
+            if (whole - k > 2 * KS * U)
+                load(0, k + 2 * KS * U);
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 mm(fa[1][u], fb[1][u]);
@@ -396,23 +404,22 @@ __global__ void __launch_bounds__(64 * kSmWaves) k_gemm_f32_small(f32_args g)
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 mm(fa[0][u], fb[0][u]);
-            k += 8 * U;
+            k += KS * U;
         }
     }
-    for (; k < kend; k += 8)
+    for (; k < kend; k += KS)
         mm(load_k4<TA>(A, g.lda, row, k + kh, kend, g.va), load_k4<!TB>(B, g.ldb, col, k + kh, kend, g.vb));
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-        part[wave][(e >> 2) * 8 + (lane >> 5) * 4 + (e & 3)][lane & 31] = acc[e];
+    for (int e = 0; e < T * T / 64; ++e)
+        part[wave][(e >> 2) * 8 + lane / T * 4 + (e & 3)][lane % T] = acc[e];
     __syncthreads();
-    const int c = tid & 31;
+    const int c = tid % T;
     if (n0 + c >= g.n)
         return;
 #pragma unroll
-    for (int u = 0; u < 1024 / (64 * kSmWaves); ++u) {
-        const int r = (tid >> 5) + u * (2 * kSmWaves);
+    for (int r = tid / T; r < T; r += 64 * kSmWaves / T) {
         if (m0 + r >= g.m)
-            continue;
+            break;
         float v = 0.0f;
 #pragma unroll
         for (int w = 0; w < kSmWaves; ++w)
@@ -420,6 +427,13 @@ __global__ void __launch_bounds__(64 * kSmWaves) k_gemm_f32_small(f32_args g)
         float *p = C + (size_t)(m0 + r) * g.ldc + n0 + c;
         *p = g.beta ? *p + v : v;
     }
+}
+
+template <int T, bool TA, bool TB>
+__global__ void __launch_bounds__(64 * kSmWaves) k_gemm_f32_small(f32_args g)
+{
+    __shared__ float part[kSmWaves][T][T + 1];
+    f32_small_block<T, TA, TB>(g, xcd_tile((int)blockIdx.x, (int)gridDim.x), part);
 }
 
 template <int BM, int BN, int WGM, int WGN, int KB, int KG, bool VEC>
@@ -445,15 +459,16 @@ void launch_tiled(int ta, int tb, f32_args g, unsigned batch, hipStream_t s)
         launch_tiled_v<BM, BN, WGM, WGN, KB, KG, false>(ta, tb, g, grid, s);
 }
 
+template <int T>
 void launch_small(int ta, int tb, f32_args g, unsigned batch, hipStream_t s)
 {
-    g.tiles_n = (g.n + 31) / 32;
-    const dim3 grid((unsigned)((g.m + 31) / 32) * (unsigned)g.tiles_n, 1, batch), block(64 * kSmWaves);
+    g.tiles_n = (g.n + T - 1) / T;
+    const dim3 grid((unsigned)((g.m + T - 1) / T) * (unsigned)g.tiles_n, 1, batch), block(64 * kSmWaves);
     switch ((ta ? 2 : 0) | (tb ? 1 : 0)) {
-    case 0: hipLaunchKernelGGL((k_gemm_f32_small<false, false>), grid, block, 0, s, g); break;
-    case 1: hipLaunchKernelGGL((k_gemm_f32_small<false, true>), grid, block, 0, s, g); break;
-    case 2: hipLaunchKernelGGL((k_gemm_f32_small<true, false>), grid, block, 0, s, g); break;
-    default: hipLaunchKernelGGL((k_gemm_f32_small<true, true>), grid, block, 0, s, g); break;
+    case 0: hipLaunchKernelGGL((k_gemm_f32_small<T, false, false>), grid, block, 0, s, g); break;
+    case 1: hipLaunchKernelGGL((k_gemm_f32_small<T, false, true>), grid, block, 0, s, g); break;
+    case 2: hipLaunchKernelGGL((k_gemm_f32_small<T, true, false>), grid, block, 0, s, g); break;
+    default: hipLaunchKernelGGL((k_gemm_f32_small<T, true, true>), grid, block, 0, s, g); break;
     }
 }
 
@@ -475,14 +490,19 @@ extern "C" int pgk_gemm_f32(int ta, int tb, size_t m, size_t n, size_t k, const 
     // faster but leaves the CU short of waves), in units of 39 us at k = 1024.
     // Measured there: 128 x 128 tiles 137 and 95 us, 64 x 64 tiles 39 and
     // 28 us (33 with one wave group), 32 x 32 tiles with the reduction split
-    // over the waves 25 and 14 us
+    // over the waves 25 and 14 us.
+    // The last take 16 x 16 tiles while those are at most 1024, four blocks
+    // per CU: 512 x 512 x 512 takes 9 us either way, smaller outputs 7 - 9
+    // against 7 - 21 us, 784 x 512 x 256 (1568 blocks) 10 against 8 us
     auto cost = [&](size_t tile, double full, double half) {
         const size_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * batch, rem = tiles % 512;
         return (double)(tiles / 512) * full + (rem > 256 ? full : rem ? half : 0.0);
     };
     const double big = cost(128, 3.5, 2.4), mid = cost(64, 1.0, 0.7), small = cost(32, 0.64, 0.36);
-    if (small <= mid && small <= big)
-        launch_small(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+    if (small <= mid && small <= big && ((m + 15) / 16) * ((n + 15) / 16) * batch <= 1024)
+        launch_small<16>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+    else if (small <= mid && small <= big)
+        launch_small<32>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
     else if (mid <= big && ((m + 63) / 64) * ((n + 63) / 64) * batch <= 256)
         launch_tiled<64, 64, 2, 2, 64, 2>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
     else if (mid <= big)

@@ -29,9 +29,11 @@ def gemm(lib):
     return f
 
 
-# (m, n, k, batch): one 32-tile and its edges, reductions shorter than a wave's
-# share, k not a multiple of 4, 8 or 64; 64-tiles from 176 of them up; 128-tiles
+# (m, n, k, batch): one 16-tile and its edges, reductions shorter than a wave's
+# share, k not a multiple of 4, 8, 16 or 64; 1024 16-tiles, and 32-tiles past
+# them; 64-tiles from 176 of them up; 128-tiles
 SHAPES = [(1, 1, 1, 1), (1, 33, 7, 3), (31, 32, 64, 1), (33, 65, 513, 2), (10, 16, 2049, 1),
+          (512, 509, 150, 1), (545, 515, 131, 1), (512, 544, 300, 1),
           (1025, 769, 64, 1), (1024, 1024, 63, 1), (1020, 772, 132, 2), (65, 64, 130, 130),
           (2944, 2945, 33, 1), (3072, 3072, 68, 1), (5, 9, 0, 2)]
 
