@@ -299,6 +299,14 @@ void pgm_matmul_backward(pg_node *n)
         if (!a32 || !b32)
             return;
         const float *gp = g->dev;
+        /* x.x has one grad, which the second product adds to: in order then,
+         * never side by side */
+        const bool both = ga && gb && B == 1 && ga != gb && ga->data_ref != gb->data_ref;
+        int rc = both ? pgk_gemm_f32_pair(M, N, K, a32, b32, gp, ga->dev, ba, gb->dev, bbeta, st) : PGK_GEMM_NOT_PAIRED;
+        if (rc != PGK_GEMM_NOT_PAIRED) {
+            pgd_check(rc, "matmul dgrad + wgrad");
+            ga = gb = NULL;
+        }
         if (ga) { /* dA[i,p] = sum_j g[i,j] B[p,j] */
             const size_t step = s.abat ? 65535 : 1; /* an unbatched A accumulates over the batch */
             for (size_t z = 0; z < B; z += step)

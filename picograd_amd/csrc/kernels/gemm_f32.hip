@@ -436,6 +436,19 @@ __global__ void __launch_bounds__(64 * kSmWaves) k_gemm_f32_small(f32_args g)
     f32_small_block<T, TA, TB>(g, xcd_tile((int)blockIdx.x, (int)gridDim.x), part);
 }
 
+// A dgrad d (A K-contiguous, B transposed) and a wgrad w (A transposed) in one
+// grid: d's blocks, then w's
+template <int T>
+__global__ void __launch_bounds__(64 * kSmWaves) k_gemm_f32_small_pair(f32_args d, f32_args w, int nd)
+{
+    __shared__ float part[kSmWaves][T][T + 1];
+    const int pid = (int)blockIdx.x;
+    if (pid < nd)
+        f32_small_block<T, false, true>(d, xcd_tile(pid, nd), part);
+    else
+        f32_small_block<T, true, false>(w, xcd_tile(pid - nd, (int)gridDim.x - nd), part);
+}
+
 template <int BM, int BN, int WGM, int WGN, int KB, int KG, bool VEC>
 void launch_tiled_v(int ta, int tb, const f32_args &g, dim3 grid, hipStream_t s)
 {
@@ -472,6 +485,50 @@ void launch_small(int ta, int tb, f32_args g, unsigned batch, hipStream_t s)
     }
 }
 
+size_t tiles_of(size_t m, size_t n, size_t batch, size_t t)
+{
+    return ((m + t - 1) / t) * ((n + t - 1) / t) * batch;
+}
+
+// The tile side of the split-over-waves kernel (16, 32), or of the tiled one
+// (64, 128): the shortest of three plans, as rounds of two blocks per CU, a
+// round of 512 blocks and one of at most 256 (one per CU, which runs a block
+// faster but leaves the CU short of waves), in units of 39 us at k = 1024.
+// Measured there: 128 x 128 tiles 137 and 95 us, 64 x 64 tiles 39 and 28 us
+// (33 with one wave group), 32 x 32 tiles with the reduction split over the
+// waves 25 and 14 us.  The last become 16 x 16 tiles while those are at most
+// kSm16Max, four blocks per CU: 512 x 512 x 512 takes 9 us either way, smaller
+// outputs 7 - 9 against 7 - 21 us, 784 x 512 x 256 (1568 blocks) 10 against 8.
+constexpr size_t kSm16Max = 1024;
+int tile_plan(size_t m, size_t n, size_t batch)
+{
+    auto cost = [&](size_t tile, double full, double half) {
+        const size_t tiles = tiles_of(m, n, batch, tile), rem = tiles % 512;
+        return (double)(tiles / 512) * full + (rem > 256 ? full : rem ? half : 0.0);
+    };
+    const double big = cost(128, 3.5, 2.4), mid = cost(64, 1.0, 0.7), small = cost(32, 0.64, 0.36);
+    if (small <= mid && small <= big)
+        return tiles_of(m, n, batch, 16) <= kSm16Max ? 16 : 32;
+    return mid <= big ? 64 : 128;
+}
+
+// 16-byte loads hold for an operand whose fragments start on 16 bytes
+// (K-contiguous: every row; MN-contiguous: every k, over whole 4-row groups)
+int vec_ok(const float *p, size_t ld, size_t stride, bool mn, size_t rows)
+{
+    return !(((uintptr_t)p & 15) | (ld & 3) | (stride & 3) | (mn ? rows & 3 : 0));
+}
+
+template <int T>
+void launch_pair(f32_args d, f32_args w, hipStream_t s)
+{
+    d.tiles_n = (d.n + T - 1) / T;
+    w.tiles_n = (w.n + T - 1) / T;
+    const unsigned nd = (unsigned)((d.m + T - 1) / T) * (unsigned)d.tiles_n,
+                   nw = (unsigned)((w.m + T - 1) / T) * (unsigned)w.tiles_n;
+    hipLaunchKernelGGL(k_gemm_f32_small_pair<T>, dim3(nd + nw), dim3(64 * kSmWaves), 0, s, d, w, (int)nd);
+}
+
 } // namespace
 
 extern "C" int pgk_gemm_f32(int ta, int tb, size_t m, size_t n, size_t k, const float *a, size_t lda,
@@ -482,32 +539,38 @@ extern "C" int pgk_gemm_f32(int ta, int tb, size_t m, size_t n, size_t k, const 
         return 0;
     if (batch > 65535 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff)
         return (int)hipErrorInvalidValue;
-    const int va = !(((uintptr_t)a & 15) | (lda & 3) | (stride_a & 3) | (ta ? m & 3 : 0));
-    const int vb = !(((uintptr_t)b & 15) | (ldb & 3) | (stride_b & 3) | (tb ? 0 : n & 3));
-    const f32_args g = {a, lda, stride_a, b, ldb, stride_b, c, ldc, stride_c, (int)m, (int)n, (int)k, beta, 0, va, vb};
-    // the shortest of three plans: rounds of two blocks per CU, a round of
-    // 512 blocks and one of at most 256 (one per CU, which runs a block
-    // faster but leaves the CU short of waves), in units of 39 us at k = 1024.
-    // Measured there: 128 x 128 tiles 137 and 95 us, 64 x 64 tiles 39 and
-    // 28 us (33 with one wave group), 32 x 32 tiles with the reduction split
-    // over the waves 25 and 14 us.
-    // The last take 16 x 16 tiles while those are at most 1024, four blocks
-    // per CU: 512 x 512 x 512 takes 9 us either way, smaller outputs 7 - 9
-    // against 7 - 21 us, 784 x 512 x 256 (1568 blocks) 10 against 8 us
-    auto cost = [&](size_t tile, double full, double half) {
-        const size_t tiles = ((m + tile - 1) / tile) * ((n + tile - 1) / tile) * batch, rem = tiles % 512;
-        return (double)(tiles / 512) * full + (rem > 256 ? full : rem ? half : 0.0);
-    };
-    const double big = cost(128, 3.5, 2.4), mid = cost(64, 1.0, 0.7), small = cost(32, 0.64, 0.36);
-    if (small <= mid && small <= big && ((m + 15) / 16) * ((n + 15) / 16) * batch <= 1024)
-        launch_small<16>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
-    else if (small <= mid && small <= big)
-        launch_small<32>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
-    else if (mid <= big && ((m + 63) / 64) * ((n + 63) / 64) * batch <= 256)
-        launch_tiled<64, 64, 2, 2, 64, 2>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
-    else if (mid <= big)
-        launch_tiled<64, 64, 2, 2, 64>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+    const f32_args g = {a, lda, stride_a, b, ldb, stride_b, c, ldc, stride_c, (int)m, (int)n, (int)k, beta, 0,
+                        vec_ok(a, lda, stride_a, ta, m), vec_ok(b, ldb, stride_b, !tb, n)};
+    switch (tile_plan(m, n, batch)) {
+    case 16: launch_small<16>(ta, tb, g, (unsigned)batch, (hipStream_t)s); break;
+    case 32: launch_small<32>(ta, tb, g, (unsigned)batch, (hipStream_t)s); break;
+    case 64:
+        if (tiles_of(m, n, batch, 64) <= 256)
+            launch_tiled<64, 64, 2, 2, 64, 2>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+        else
+            launch_tiled<64, 64, 2, 2, 64>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+        break;
+    default: launch_tiled<128, 128, 2, 2, 32>(ta, tb, g, (unsigned)batch, (hipStream_t)s); break;
+    }
+    return (int)hipGetLastError();
+}
+
+// Both on the split-over-waves kernel when each alone would be: a launch
+// boundary (about 1.2 us between dependent kernels) less, and the blocks of
+// the one fill the CUs that the other leaves idle
+extern "C" int pgk_gemm_f32_pair(size_t m, size_t n, size_t k, const float *a, const float *b, const float *g,
+                                 float *da, int beta_a, float *db, int beta_b, pgk_stream s)
+{
+    if (!m || !n || !k || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff || tile_plan(m, k, 1) > 32 ||
+        tile_plan(k, n, 1) > 32)
+        return PGK_GEMM_NOT_PAIRED;
+    const f32_args d = {g, n, 0, b, n, 0, da, k, 0, (int)m, (int)k, (int)n, beta_a, 0, vec_ok(g, n, 0, false, m),
+                        vec_ok(b, n, 0, false, k)};
+    const f32_args w = {a, k, 0, g, n, 0, db, n, 0, (int)k, (int)n, (int)m, beta_b, 0, vec_ok(a, k, 0, true, k),
+                        vec_ok(g, n, 0, true, n)};
+    if (tiles_of(m, k, 1, 16) + tiles_of(k, n, 1, 16) <= kSm16Max)
+        launch_pair<16>(d, w, (hipStream_t)s);
     else
-        launch_tiled<128, 128, 2, 2, 32>(ta, tb, g, (unsigned)batch, (hipStream_t)s);
+        launch_pair<32>(d, w, (hipStream_t)s);
     return (int)hipGetLastError();
 }

@@ -211,6 +211,12 @@ int pgk_mfma_probe(int lds, float *sink, size_t sink_floats, int blocks, int ite
 int pgk_gemm_f32(int ta, int tb, size_t m, size_t n, size_t k, const float *a, size_t lda,
                  size_t stride_a, const float *b, size_t ldb, size_t stride_b, float *c,
                  size_t ldc, size_t stride_c, size_t batch, int beta, pgk_stream s);
+/* Both grads of c = a b (a [m, k], b [k, n], g = dc [m, n], all dense) in one
+ * launch when both are small: da (beta_a ? += : =) g b^T, db (beta_b ? += : =)
+ * a^T g.  PGK_GEMM_NOT_PAIRED (nothing launched) otherwise.  da and db must
+ * not overlap. */
+int pgk_gemm_f32_pair(size_t m, size_t n, size_t k, const float *a, const float *b, const float *g, float *da,
+                      int beta_a, float *db, int beta_b, pgk_stream s);
 
 /* The last step of a bias grad: out[c] (beta ? += : =) the sum over the
  * nblk row-block partials part[b * n + c], b in order. */

@@ -126,3 +126,61 @@ def test_matmul_f32_batched_backward(lib, abat, bbat):
     lib.pg_tensor_free(tg)
     lib.pg_node_free(na)
     lib.pg_node_free(nw)
+
+
+# (m, k, n) around what one launch holds: 16-tiles up to 1024 of them in all,
+# odd and even rows, more of them (32-tiles), and a pair that is too large
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (17, 33, 10), (200, 20, 1001), (256, 256, 512), (260, 500, 300),
+                                   (640, 784, 512), (1300, 1100, 65)])
+@pytest.mark.parametrize("beta", [0, 1])
+def test_matmul_f32_backward_pair(lib, gemm, m, k, n, beta):
+    """Both grads of a product in one launch against f64, and against the two
+    launches they replace; C of neither reaches past its own elements."""
+    f = lib.lib.pgk_gemm_f32_pair
+    sz, vp = C.c_size_t, C.c_void_p
+    f.restype, f.argtypes = C.c_int, [sz, sz, sz, vp, vp, vp, vp, C.c_int, vp, C.c_int, vp]
+    rng = np.random.default_rng(m + 3 * k + 5 * n)
+    a, b, g = (rng.standard_normal(s).astype(np.float32) for s in ((m, k), (k, n), (m, n)))
+    a64, b64, g64 = (x.astype(np.float64) for x in (a, b, g))
+    ta, tb, tg = lib.tensor(a), lib.tensor(b), lib.tensor(g)
+    pa, pb, pg = (lib.tinfo(t).dev for t in (ta, tb, tg))
+    c0 = [np.full(r * c + 64, SENTINEL, np.float32) for r, c in ((m, k), (k, n))]
+    for x, size in zip(c0, (m * k, k * n)):
+        x[:size] = rng.standard_normal(size)
+    one, two = [lib.tensor(x) for x in c0], [lib.tensor(x) for x in c0]
+    st = lib.pg_amd_stream()
+    rc = f(m, n, k, pa, pb, pg, lib.tinfo(one[0]).dev, beta, lib.tinfo(one[1]).dev, 1 - beta, st)
+    assert rc == (-1 if m == 1300 else 0)
+    assert gemm(0, 1, m, k, n, pg, n, 0, pb, n, 0, lib.tinfo(two[0]).dev, k, 0, 1, beta, st) == 0
+    assert gemm(1, 0, k, n, m, pa, k, 0, pg, n, 0, lib.tinfo(two[1]).dev, n, 0, 1, 1 - beta, st) == 0
+    refs = ((g64 @ b64.T, np.abs(g64) @ np.abs(b64.T), n, beta), (a64.T @ g64, np.abs(a64.T) @ np.abs(g64), m, 1 - beta))
+    for t, t2, x, (ref, mag, red, bt) in zip(one, two, c0, refs):
+        got, got2 = lib.read(t), lib.read(t2)
+        size = ref.size
+        if rc:
+            assert np.array_equal(got, x)
+            got = got2
+        base = x[:size].astype(np.float64) * bt
+        bound = gamma(red + 2) * (mag.reshape(-1) + np.abs(base)) + 1e-38
+        for y in (got, got2):
+            assert (np.abs(y[:size] - (ref.reshape(-1) + base)) <= bound).all()
+            assert (y[size:] == SENTINEL).all()
+    for t in (ta, tb, tg, *one, *two):
+        lib.pg_tensor_free(t)
+
+
+def test_matmul_f32_backward_shared_operand(lib):
+    """x x has one grad, the sum of both products: never written side by side."""
+    n = 96
+    x = np.random.default_rng(3).standard_normal((n, n)).astype(np.float32)
+    g = np.random.default_rng(4).standard_normal((n, n)).astype(np.float32)
+    nx, tg = lib.var(x), lib.tensor(g)
+    y = lib.op("matmul", nx, nx)
+    x64, g64 = x.astype(np.float64), g.astype(np.float64)
+    mag = np.abs(g64) @ np.abs(x64.T) + np.abs(x64.T) @ np.abs(g64)
+    for _ in range(2):
+        lib.pg_amd_backward_from(y, tg)
+        assert (np.abs(lib.grad(nx) - (g64 @ x64.T + x64.T @ g64)) <= gamma(n + 3) * mag).all()
+    lib.pg_node_free(y)
+    lib.pg_tensor_free(tg)
+    lib.pg_node_free(nx)
