@@ -863,6 +863,102 @@ __global__ void __launch_bounds__(kBlock) k_act_bwd16(const float *__restrict__ 
     }
 }
 
+// The same pass with the bias grad whole in it, for few rows, where launches
+// and load latency are all the time: a block of 1024 lanes owns 32 columns (a
+// whole 128-byte line per row) and every row, so its column sums are db itself
+// and neither partials nor a second launch are left.  Lane (cx, ry) takes
+// columns 4 cx .. 4 cx + 3 of rows ry, ry + 128, ..., four rows' loads at
+// once; each lane's rows are added in order, then the 128 row lanes by a fixed
+// tree.  With the launch that adds the partials: 7 -> 4.5 - 5.9 us at up to
+// 256 x 4096.
+constexpr int kActColsThreads = 1024, kActColsMax = 256;
+template <int ACT, int DT>
+__global__ void __launch_bounds__(kActColsThreads)
+    k_act_bwd16_cols(const float *__restrict__ g, const float *__restrict__ z, int m, size_t n,
+                     uint16_t *__restrict__ d16, size_t ldd, float *__restrict__ db, int beta, pgk_colsum_job fin)
+{
+    constexpr int CW = 32, CL = CW / 4, RL = kActColsThreads / CL, U = 4;
+    __shared__ float red[RL][CW + 1];
+    size_t bx = blockIdx.x;
+    if (fin.part) { // as in k_act_bwd16
+        const size_t fb = (fin.n + kActColsThreads - 1) / kActColsThreads;
+        if (bx < fb) {
+            colsum_cols(fin, bx * kActColsThreads + threadIdx.x, fb * kActColsThreads);
+            return;
+        }
+        bx -= fb;
+    }
+    const int cx = threadIdx.x % CL, ry = threadIdx.x / CL;
+    const size_t c0 = bx * CW + (size_t)cx * 4;
+    const bool in = c0 < ldd;
+    const bool vec = c0 + 4 <= n && (n & 3) == 0 && ((((uintptr_t)g) | ((uintptr_t)z)) & 15) == 0;
+    float acc[4] = {};
+    for (int r0 = ry; r0 < m && in; r0 += U * RL) {
+        float gv[U][4], zv[U][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int r = r0 + u * RL;
+            const size_t off = (size_t)r * n + c0;
+            if (r < m && vec) {
+                const float4 a = ntl4(g + off);
+                gv[u][0] = a.x, gv[u][1] = a.y, gv[u][2] = a.z, gv[u][3] = a.w;
+                if (ACT) {
+                    const float4 b = ntl4(z + off);
+                    zv[u][0] = b.x, zv[u][1] = b.y, zv[u][2] = b.z, zv[u][3] = b.w;
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const bool ok = r < m && c0 + q < n;
+                    gv[u][q] = ok ? g[off + q] : 0.0f;
+                    zv[u][q] = ok && ACT ? z[off + q] : 0.0f;
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int r = r0 + u * RL;
+            if (r < m) {
+                uint32_t w[2];
+#pragma unroll
+                for (int q = 0; q < 4; q += 2) {
+#pragma clang fp contract(off)
+                    const float d0 = ACT ? gv[u][q] * act_grad(ACT, zv[u][q]) : gv[u][q];
+                    const float d1 = ACT ? gv[u][q + 1] * act_grad(ACT, zv[u][q + 1]) : gv[u][q + 1];
+                    acc[q] += d0;
+                    acc[q + 1] += d1;
+                    w[q / 2] = to16x2(DT, d0, d1);
+                }
+                *reinterpret_cast<uint2 *>(d16 + (size_t)r * ldd + c0) = make_uint2(w[0], w[1]);
+            }
+        }
+    }
+    if (!db)
+        return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        red[ry][cx * 4 + q] = acc[q];
+    // every lane adds RL / NG rows in order, then one lane per column the NG groups
+    constexpr int NG = kActColsThreads / CW;
+    const int c = threadIdx.x % CW, y = threadIdx.x / CW;
+    __syncthreads();
+    float s = 0.0f;
+#pragma unroll
+    for (int q = 0; q < RL / NG; ++q)
+        s += red[y * (RL / NG) + q][c];
+    __syncthreads();
+    red[y][c] = s;
+    __syncthreads();
+    const size_t col = bx * CW + (size_t)c;
+    if (y || col >= n)
+        return;
+    s = 0.0f;
+#pragma unroll
+    for (int q = 0; q < NG; ++q)
+        s += red[q][c];
+    db[col] = beta ? db[col] + s : s;
+}
+
 // The same pass when the grad g is itself the dgrad of a narrow next layer:
 // g = dn . wn^T with dn [m, kw] and wn [n, kw] 16-bit, kw = ldn = ldw = 8
 // or 16 (a layer of at most 16 outputs, its dz and its weights' copy with
@@ -1545,12 +1641,24 @@ extern "C" int pgk_act_bwd16(int act, const float *g, const float *z, size_t m, 
     const size_t rpb = act_bwd_rpb(m, ldd), nrb = (m + rpb - 1) / rpb;
     if (nrb + nf > 65535)
         return (int)hipErrorInvalidValue;
+    // a bias grad of up to 256 rows, in blocks of all rows while there is at
+    // most one per CU: past either, a block's serial rows cost what the second
+    // launch does (512 x 1024 and 256 x 8192 take the same 7 us both ways,
+    // 1000 x 4096 10 us in two launches and 15 in one)
+    const bool cols = db && m <= 256 && (ldd + 31) / 32 <= kActColsMax;
     const unsigned gx = (unsigned)((ldd + 127) / 128);
     float *part = db ? (float *)ws : nullptr;
     const dim3 grid(gx, (unsigned)(nrb + nf));
+    const dim3 cgrid((unsigned)((ldd + 31) / 32 + (nf ? (fin.n + kActColsThreads - 1) / kActColsThreads : 0)));
 #define PGK_ACT_BWD(A, D)                                                                                              \
-    hipLaunchKernelGGL((k_act_bwd16<A, D>), grid, dim3(kBlock), 0, (hipStream_t)s, g, z, m, n, d16, ldd, part, rpb,   \
-                       fin)
+    do {                                                                                                               \
+        if (cols)                                                                                                      \
+            hipLaunchKernelGGL((k_act_bwd16_cols<A, D>), cgrid, dim3(kActColsThreads), 0, (hipStream_t)s, g, z,        \
+                               (int)m, n, d16, ldd, db, db_beta, fin);                                                 \
+        else                                                                                                           \
+            hipLaunchKernelGGL((k_act_bwd16<A, D>), grid, dim3(kBlock), 0, (hipStream_t)s, g, z, m, n, d16, ldd, part, \
+                               rpb, fin);                                                                              \
+    } while (0)
     const bool f16 = dtype == 1;
     if (act == 0 && f16)
         PGK_ACT_BWD(0, 1);
@@ -1566,7 +1674,7 @@ extern "C" int pgk_act_bwd16(int act, const float *g, const float *z, size_t m, 
         PGK_ACT_BWD(2, 2);
 #undef PGK_ACT_BWD
     const int st = status();
-    if (st || !db)
+    if (st || !db || cols)
         return st;
     return finish_db(part, nrb, n, db, db_beta, defer, s);
 }

@@ -235,7 +235,7 @@ int pgk_colsum_run(const pgk_colsum_job *job, pgk_stream s);
  * fixed order (ws holds pgk_act_bwd16_workspace bytes): the pass writes the
  * row-block partials to ws and a second launch adds them, unless defer is
  * given, which then receives that last step as a job (ws must stay as it is
- * until the job runs).  A job given as fold (an earlier pass's deferred
+ * until the job runs; an empty job when the pass adds the whole of db).  A job given as fold (an earlier pass's deferred
  * one, its partials not in ws) runs in this pass's launch, in a row of extra
  * blocks. */
 size_t pgk_act_bwd16_workspace(size_t m, size_t n);

@@ -1,0 +1,79 @@
+"""The activation pass that holds every row of its columns (up to 256 rows, at
+most 256 blocks of 32 columns) against the one with a second launch.
+
+Its 16-bit rows must have the bits of the pass without a bias grad (which never
+takes it).  Its sums add at most 2 rows of a lane, 4 lanes, 32 groups and C, so
+they lie within gamma(40) sum |dz| of the f64 sum; dz itself is g act'(z) in f32:
+exact for none and ReLU; GELU' is a sum of two terms of order 1 that cancel near
+z = -0.75, so its error against the oracle's is 1e-6 of g, not of dz.
+"""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gemm_check import gamma
+
+pytestmark = pytest.mark.gpu
+
+SENTINEL = np.float32(-3.0e33)
+
+
+class Job(C.Structure):
+    _fields_ = [("part", C.c_void_p), ("nblk", C.c_size_t), ("n", C.c_size_t), ("out", C.c_void_p), ("beta", C.c_int)]
+
+
+# rows: less than a lane's, one and two loads per lane, the last row count it
+# takes, the first it does not; columns: below a 4-group, a 32-block's edges, odd,
+# the widest, past it
+@pytest.mark.parametrize("act", [0, 1, 2])
+@pytest.mark.parametrize("m,n", [(1, 1), (3, 33), (127, 31), (128, 64), (129, 1000), (255, 37), (256, 96), (256, 8192),
+                                 (2, 8185), (257, 40), (5, 8200)])
+def test_pass_with_whole_columns(lib, oracle, m, n, act):
+    f = lib.lib.pgk_act_bwd16
+    sz, vp = C.c_size_t, C.c_void_p
+    f.restype = C.c_int
+    f.argtypes = [C.c_int, vp, vp, sz, sz, vp, sz, C.c_int, vp, C.c_int, vp, vp, vp, vp]
+    lib.lib.pgk_act_bwd16_workspace.restype, lib.lib.pgk_act_bwd16_workspace.argtypes = sz, [sz, sz]
+    rng = np.random.default_rng(m * 11 + n + act)
+    g, z = rng.standard_normal((m, n)).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    z[0, 0] = 0.0
+    ldd = (n + 7) // 8 * 8
+    dz = [lambda: g, lambda: np.where(z > 0, g, np.float32(0)), lambda: oracle.gelu_backward(z, g).reshape(m, n)][act]()
+    tg, tz = lib.tensor(g), lib.tensor(z)
+    ws = lib.tensor(np.zeros(lib.lib.pgk_act_bwd16_workspace(m, n) // 4 + 1, np.float32))
+    db0 = np.full(n + 64, SENTINEL, np.float32)
+    db0[:n] = rng.standard_normal(n)
+    # an earlier pass's sums, finished in this one's launch
+    part = rng.standard_normal((3, 1100)).astype(np.float32)
+    tp = lib.tensor(part)
+    dev = lambda t: lib.tinfo(t).dev  # noqa: E731
+    for dt in (1, 2):
+        for beta, folds in ((0, False), (1, True)):
+            want, got = (lib.tensor(np.full(m * ldd // 2 + 64, SENTINEL, np.float32)) for _ in range(2))
+            tdb, tout = lib.tensor(db0), lib.tensor(np.full(1100, SENTINEL, np.float32))
+            st = lib.pg_amd_stream()  # after the last upload
+            fold, rest = Job(dev(tp), 3, 1100, dev(tout), 0), Job()
+            assert f(act, dev(tg), dev(tz), m, n, dev(want), ldd, dt, None, 0, None, None, None, st) == 0
+            assert f(act, dev(tg), dev(tz), m, n, dev(got), ldd, dt, dev(tdb), beta, dev(ws),
+                     C.byref(fold) if folds else None, C.byref(rest), st) == 0
+            assert bool(rest.part) == (m > 256 or n > 8192)
+            if rest.part:
+                lib.lib.pgk_colsum_run.restype, lib.lib.pgk_colsum_run.argtypes = C.c_int, [vp, vp]
+                assert lib.lib.pgk_colsum_run(C.byref(rest), st) == 0
+            assert np.array_equal(lib.read(want).view(np.uint32), lib.read(got).view(np.uint32))
+            out = lib.read(tdb)
+            ref, mag = dz.astype(np.float64).sum(0), np.abs(dz.astype(np.float64)).sum(0)
+            base = db0[:n].astype(np.float64) * beta
+            depth = 40 if not rest.part else 128
+            form = 1e-6 * np.abs(g.astype(np.float64)).sum(0) if act == 2 else 0.0
+            bound = gamma(depth) * mag + form + gamma(2) * np.abs(base) + 1e-30
+            assert (np.abs(out[:n] - (ref + base)) <= bound).all()
+            assert (out[n:] == SENTINEL).all()
+            assert np.array_equal(lib.read(tout), part[0] + part[1] + part[2] if folds else np.full(1100, SENTINEL))
+            for t in (want, got, tdb, tout):
+                lib.pg_tensor_free(t)
+    for t in (tg, tz, ws, tp):
+        lib.pg_tensor_free(t)
