@@ -166,6 +166,31 @@ static bool pair_ks(int dt, const pgk_gemm_desc *dd, const pgk_gemm_desc *dw, co
     return pgd_check(rc, what);
 }
 
+/* The CUs that dgrad [M, K] (reduction N8) should take of the chip, wgrad
+ * [K, N] (reduction Mw) beside it on the rest, 0 when the two run one after
+ * the other: by the planner's estimates, with a clear win.  *streams: whether
+ * two streams may do it where one launch cannot hold both.  Not for a problem
+ * whose own plan is a split-over-waves tile or the few-rows kernel: those take
+ * a few us where the fork and join of a second stream take about 30 (f16 forward
+ * and grads of 118 x 2275 x 11: 35 us one after the other, 70 on two streams;
+ * 32 x 1439 x 47 in 15 batches: 39 and 68). */
+int pgm_grad_split(size_t M, size_t K, size_t N, size_t N8, size_t B, size_t Mw, size_t Bw, bool *streams)
+{
+    *streams = pgk_gemm16_plan(0, 0, M, K, N8, B, 0, NULL) < 5 && pgk_gemm16_plan(1, 1, K, N, Mw, Bw, 0, NULL) < 5;
+    double td = pgk_gemm16_time(0, 0, M, K, N8, B, 0), tw = pgk_gemm16_time(1, 1, K, N, Mw, Bw, 0);
+    double best = 0.85 * (td + tw);
+    int cus = 0;
+    for (int cd = 32; cd <= 224; cd += 32) {
+        double a1 = pgk_gemm16_time(0, 0, M, K, N8, B, cd), a2 = pgk_gemm16_time(1, 1, K, N, Mw, Bw, 256 - cd);
+        double t = a1 > a2 ? a1 : a2;
+        if (t < best) {
+            best = t;
+            cus = cd;
+        }
+    }
+    return cus;
+}
+
 /* 16-bit copy of `rows x cols` (leading dim lds, `batch` matrices `sstride`
  * apart) padded with zeros to rows_pad x cols_pad; src_dtype 0 casts f32 */
 static uint16_t *stage16(int dt, int src_dtype, const void *src, size_t rows, size_t cols, size_t lds,
@@ -386,22 +411,13 @@ void pgm_matmul_backward(pg_node *n)
         return;
     }
     if (d_one && w_one && !alias) {
-        double td = pgk_gemm16_time(0, 0, M, K, N8, B, 0), tw = pgk_gemm16_time(1, 1, K, N, Mw, Bw, 0);
-        double best = 0.85 * (td + tw);
-        int best_cus = 0;
-        for (int cd = 32; cd <= 224; cd += 32) {
-            double a1 = pgk_gemm16_time(0, 0, M, K, N8, B, cd), a2 = pgk_gemm16_time(1, 1, K, N, Mw, Bw, 256 - cd);
-            double t = a1 > a2 ? a1 : a2;
-            if (t < best) {
-                best = t;
-                best_cus = cd;
-            }
-        }
+        bool streams;
+        const int best_cus = pgm_grad_split(M, K, N, N8, B, Mw, Bw, &streams);
         if (best_cus) {
             tk = pgd_tbegin(PGD_T_GEMM16); /* the pair is one interval */
             pd.timed = pw.timed = false;
             /* one launch holding both when it can (no second stream to
-             * fork and join), else the two on two streams */
+             * fork and join), else the two on two streams or in turn */
             size_t offw = 0, wsz = pgk_gemm16_pair_dw_workspace(&dd, &dw, best_cus, &offw);
             void *ws = wsz ? pgd_scratch(1, wsz) : NULL;
             int rc = wsz && !ws ? PGK_GEMM_NOT_PAIRED : pgk_gemm16_pair_dw(dt, &dd, &dw, best_cus, ws, pgd_stream());
@@ -419,7 +435,7 @@ void pgm_matmul_backward(pg_node *n)
              * growing it afterwards would reuse a freed block in main-stream
              * order, which the side stream does not follow */
             size_t w5 = pgk_gemm16_workspace_cu(1, 1, K, N, Mw, Bw, 256 - best_cus);
-            pgk_stream side = !w5 || pgd_scratch(5, w5) ? pgd_fork() : NULL;
+            pgk_stream side = streams && (!w5 || pgd_scratch(5, w5)) ? pgd_fork() : NULL;
             if (side) {
                 pd.cus = best_cus;
                 pw = (gemm_place){side, 5, 256 - best_cus, false};

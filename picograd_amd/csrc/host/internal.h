@@ -186,6 +186,7 @@ pg_tensor *pgm_matmul_forward(const pg_tensor *a, const pg_tensor *b);
  * storage replaces its staging pass), else 0 */
 int pgm_mm16_grad16(const pg_node *n);
 void pgm_matmul_backward(pg_node *n);
+int pgm_grad_split(size_t M, size_t K, size_t N, size_t N8, size_t B, size_t Mw, size_t Bw, bool *streams);
 /* a linear16 bias grad whose last step (the sum of its row-block partials)
  * the next activation pass was to run: run it now (the walk's end), or now
  * if it writes into t's storage (t is about to be written) */

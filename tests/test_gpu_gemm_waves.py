@@ -123,7 +123,28 @@ def test_pair_in_one_launch(lib, oracle, k, shape, dt):  # noqa: F811
     check_product(aw[GUARD:GUARD + K, :N], [(f(X).T, f(G))], what + " dW", add=c0w)
 
 
-@pytest.mark.parametrize("batch,M,K,N", [(3, 65, 24, 40), (2, 200, 72, 136), (24, 64, 64, 128)])
+@pytest.mark.parametrize("M,K,N", [(30, 1202, 10), (118, 2275, 11)])
+def test_matmul_with_small_grads(lib, oracle, M, K, N):
+    """Grads that no one launch holds and that run one after the other."""
+    print(f"waves matmul {M}x{K}x{N}", flush=True)
+    rng = np.random.default_rng(M)
+    a = oracle.cast16(F16, rng.standard_normal((M, K)).astype(np.float32))
+    b = oracle.cast16(F16, rng.standard_normal((K, N)).astype(np.float32))
+    g = _f32(F16, oracle.cast16(F16, rng.standard_normal((M, N)).astype(np.float32)))
+    na, nb, tg = lib.var(a, dtype=F16), lib.var(b, dtype=F16), lib.tensor(g)
+    y = lib.op("matmul", na, nb)
+    lib.pg_amd_backward_from(y, tg)
+    fa, fb = _f32(F16, a), _f32(F16, b)
+    check_product(lib.value(y), [(fa, fb)], "forward")
+    check_product(lib.grad(na), [(g, fb.T)], "dA")
+    check_product(lib.grad(nb), [(fa.T, g)], "dB")
+    lib.pg_node_free(y)
+    lib.pg_tensor_free(tg)
+    lib.pg_node_free(na)
+    lib.pg_node_free(nb)
+
+
+@pytest.mark.parametrize("batch,M,K,N", [(3, 65, 24, 40), (2, 200, 72, 136), (24, 64, 64, 128), (15, 32, 1439, 47)])
 def test_batched_matmul(lib, oracle, batch, M, K, N):
     """pg_ag_matmul over batches: forward and both grads, each entry's own."""
     dt = F16
