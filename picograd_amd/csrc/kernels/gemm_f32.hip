@@ -557,18 +557,34 @@ extern "C" int pgk_gemm_f32(int ta, int tb, size_t m, size_t n, size_t k, const 
 
 // Both on the split-over-waves kernel when each alone would be: a launch
 // boundary (about 1.2 us between dependent kernels) less, and the blocks of
-// the one fill the CUs that the other leaves idle
-extern "C" int pgk_gemm_f32_pair(size_t m, size_t n, size_t k, const float *a, const float *b, const float *g,
-                                 float *da, int beta_a, float *db, int beta_b, pgk_stream s)
+// the one fill the CUs that the other leaves idle.  Not when the shared tile
+// is 32 x 32 and one of them would alone be at most 256 tiles of 16 x 16 over
+// a reduction of more than 640: the larger tile's chain of load latencies then
+// costs more than the launch (8192 x 64 x 64: 79 us in one launch, 26 in two;
+// 752 x 424 x 66: 11.0 and 9.7), and up to there less (437 x 613 x 56: 7.2 and
+// 8.5 us; 540 tiles at 711 x 189 x 1293: 27 and 37).
+extern "C" int pgk_gemm_f32_pair_tile(size_t m, size_t n, size_t k)
 {
     if (!m || !n || !k || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff || tile_plan(m, k, 1) > 32 ||
         tile_plan(k, n, 1) > 32)
+        return 0;
+    const size_t td = tiles_of(m, k, 1, 16), tw = tiles_of(k, n, 1, 16);
+    if (td + tw <= kSm16Max)
+        return 16;
+    return (td <= 256 && n > 640) || (tw <= 256 && m > 640) ? 0 : 32;
+}
+
+extern "C" int pgk_gemm_f32_pair(size_t m, size_t n, size_t k, const float *a, const float *b, const float *g,
+                                 float *da, int beta_a, float *db, int beta_b, pgk_stream s)
+{
+    const int tile = pgk_gemm_f32_pair_tile(m, n, k);
+    if (!tile)
         return PGK_GEMM_NOT_PAIRED;
     const f32_args d = {g, n, 0, b, n, 0, da, k, 0, (int)m, (int)k, (int)n, beta_a, 0, vec_ok(g, n, 0, false, m),
                         vec_ok(b, n, 0, false, k)};
     const f32_args w = {a, k, 0, g, n, 0, db, n, 0, (int)k, (int)n, (int)m, beta_b, 0, vec_ok(a, k, 0, true, k),
                         vec_ok(g, n, 0, true, n)};
-    if (tiles_of(m, k, 1, 16) + tiles_of(k, n, 1, 16) <= kSm16Max)
+    if (tile == 16)
         launch_pair<16>(d, w, (hipStream_t)s);
     else
         launch_pair<32>(d, w, (hipStream_t)s);

@@ -214,7 +214,8 @@ int pgk_gemm_f32(int ta, int tb, size_t m, size_t n, size_t k, const float *a, s
 /* Both grads of c = a b (a [m, k], b [k, n], g = dc [m, n], all dense) in one
  * launch when both are small: da (beta_a ? += : =) g b^T, db (beta_b ? += : =)
  * a^T g.  PGK_GEMM_NOT_PAIRED (nothing launched) otherwise.  da and db must
- * not overlap. */
+ * not overlap.  _tile: the tile side both take, 0 when they are not paired. */
+int pgk_gemm_f32_pair_tile(size_t m, size_t n, size_t k);
 int pgk_gemm_f32_pair(size_t m, size_t n, size_t k, const float *a, const float *b, const float *g, float *da,
                       int beta_a, float *db, int beta_b, pgk_stream s);
 

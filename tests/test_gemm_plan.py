@@ -1,5 +1,5 @@
-"""The GEMM planner's choices, which need no device: when the two grads of a
-matmul may run on two streams."""
+"""The GEMM planner's choices, which need no device: which f32 grads
+share a launch, and when the two grads of a matmul may run on two streams."""
 from __future__ import annotations
 
 import ctypes as C
@@ -16,6 +16,14 @@ def k():
     lib.pgk_gemm16_plan.restype, lib.pgk_gemm16_plan.argtypes = i, [i, i, sz, sz, sz, sz, i, C.POINTER(i)]
     lib.pgm_grad_split.restype, lib.pgm_grad_split.argtypes = i, [sz] * 7 + [C.POINTER(C.c_bool)]
     return lib
+
+
+@pytest.mark.parametrize("m,kk,n,tile", [(8192, 64, 64, 0), (16384, 64, 64, 0), (2048, 256, 256, 0), (752, 424, 66, 0),
+                                         (45, 270, 985, 0), (437, 613, 56, 32), (711, 189, 1293, 32),
+                                         (256, 784, 512, 32), (256, 256, 512, 16)])
+def test_f32_pairs_decline_a_long_reduction_on_the_larger_tile(k, m, kk, n, tile):
+    k.pgk_gemm_f32_pair_tile.restype, k.pgk_gemm_f32_pair_tile.argtypes = C.c_int, [C.c_size_t] * 3
+    assert k.pgk_gemm_f32_pair_tile(m, n, kk) == tile
 
 
 @pytest.mark.parametrize("M,K,N,B,two", [
