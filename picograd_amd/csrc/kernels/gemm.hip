@@ -859,20 +859,27 @@ __device__ __forceinline__ void ks_block(const gemm_kargs &g, int has_epi, int p
                 OB::load_q(q, B, g.ldb, n0, g.b_extent, k0, g.K, sb, lane);
         }
     };
-    f32x16 acc[FM][FN];
+    // Four waves keep two sums each, their even and odd chunks': eight partial
+    // sums of a reduction, as many as eight waves or the split-K plan have, so
+    // the error against 64 bits is no larger than theirs (dW of 2048 x 512 x 512:
+    // 1.02e-7, with one sum per wave 1.32e-7)
+    constexpr int NA = KG == 4 ? 2 : 1;
+    f32x16 acc[NA][FM][FN];
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int a = 0; a < NA; ++a)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-                acc[i][j][e] = 0.0f;
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    acc[a][i][j][e] = 0.0f;
     if (nc > 0) {
 #pragma unroll
         for (int s = 0; s < S; ++s)
             load(s, s);
         int st = 0;
-        for (int c = 0; c < nc; ++c) {
+        auto chunk = [&](int c, f32x16(&sum)[FM][FN]) {
             const LDS uint4 *sa = ring + st * CF::STAGE, *sb = sa + SA;
             // chunk c landed (the newest S - 1 chunks may be in flight)
             __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm((S - 1) * LPT));
@@ -897,11 +904,25 @@ __device__ __forceinline__ void ks_block(const gemm_kargs &g, int has_epi, int p
                 for (int i = 0; i < FM; ++i)
 #pragma unroll
                     for (int j = 0; j < FN; ++j)
-                        acc[i][j] = mfma32<F16>(fa[s][i], fb[s][j], acc[i][j]);
+                        sum[i][j] = mfma32<F16>(fa[s][i], fb[s][j], sum[i][j]);
             st = st + 1 == S ? 0 : st + 1;
-        }
+        };
+        int c = 0;
+        for (; c + NA <= nc; c += NA)
+#pragma unroll
+            for (int a = 0; a < NA; ++a)
+                chunk(c + a, acc[a]);
+        if (c < nc) // NA == 2: the last even chunk
+            chunk(c, acc[0]);
         __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(0));
     }
+#pragma unroll
+    for (int a = 1; a < NA; ++a)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                acc[0][i][j] += acc[a][i][j];
     __syncthreads(); // the rings are done
     LDS float *part = (LDS float *)lds;
     const int lrow = lane & 31, lk = lane >> 5;
@@ -911,7 +932,7 @@ __device__ __forceinline__ void ks_block(const gemm_kargs &g, int has_epi, int p
         for (int j = 0; j < FN; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e)
-                part[(wave * TM + i * 32 + (e >> 2) * 8 + lk * 4 + (e & 3)) * CF::RS + j * 32 + lrow] = acc[i][j][e];
+                part[(wave * TM + i * 32 + (e >> 2) * 8 + lk * 4 + (e & 3)) * CF::RS + j * 32 + lrow] = acc[0][i][j][e];
     __syncthreads();
     float *C = g.C + (size_t)z * g.sC;
     const pgk_epi &epi = g.epi;
@@ -956,8 +977,9 @@ __device__ __forceinline__ void ks_block(const gemm_kargs &g, int has_epi, int p
     }
 }
 
+// four-wave blocks stay within two waves per SIMD, so two blocks share a CU
 template <class CF>
-__global__ void __launch_bounds__(CF::NT, 1) k_gemm16_ks(gemm_kargs g, int has_epi)
+__global__ void __launch_bounds__(CF::NT, CF::KG == 4 ? 2 : 1) k_gemm16_ks(gemm_kargs g, int has_epi)
 {
     __shared__ uint4 smem[CF::LDS_U4];
     ks_block<CF>(g, has_epi, (int)blockIdx.x, (int)gridDim.x, true, (int)blockIdx.z, (LDS uint4 *)smem);
@@ -966,7 +988,7 @@ __global__ void __launch_bounds__(CF::NT, 1) k_gemm16_ks(gemm_kargs g, int has_e
 // a matmul's dgrad (blocks [0, n1)) and wgrad in one launch, each nb tiles
 // per batch entry, on one tile shape
 template <class C1, class C2>
-__global__ void __launch_bounds__(C1::NT, 1) k_gemm16_ks_pair(gemm_kargs g1, gemm_kargs g2, int nb1, int n1, int nb2)
+__global__ void __launch_bounds__(C1::NT, C1::KG == 4 ? 2 : 1) k_gemm16_ks_pair(gemm_kargs g1, gemm_kargs g2, int nb1, int n1, int nb2)
 {
     static_assert(C1::NT == C2::NT && C1::LDS_U4 == C2::LDS_U4, "one tile shape");
     __shared__ uint4 smem[C1::LDS_U4];

@@ -123,6 +123,42 @@ def test_pair_in_one_launch(lib, oracle, k, shape, dt):  # noqa: F811
     check_product(aw[GUARD:GUARD + K, :N], [(f(X).T, f(G))], what + " dW", add=c0w)
 
 
+@pytest.mark.parametrize("M,K,N", [(2048, 512, 512), (4096, 256, 200), (560, 488, 3312)])
+def test_pair_error_is_no_larger_than_the_split(lib, oracle, k, M, K, N):
+    """Each grad's error against f64 beside that of the plan that splits the
+    reduction over blocks (a budget of 255 CUs asks for a tiled plan): no fewer
+    partial sums.  The two errors are norms over at least 51200 independent
+    elements, so they differ by well under 5 % where the sums are alike; one sum
+    per wave measures 1.2 to 1.4 times the split's."""
+    print(f"pair error M={M} K={K} N={N}", flush=True)
+    rng = np.random.default_rng(M)
+    X, W, G = (oracle.cast16(BF16, rng.standard_normal(s).astype(np.float32)) for s in ((M, K), (K, N), (M, N)))
+    f = lambda h: _f32(BF16, h).astype(np.float64)  # noqa: E731
+    refs = f(G) @ f(W).T, f(X).T @ f(G)
+    fn = k.pgk_gemm16_ks_pair
+    fn.restype, fn.argtypes = C.c_int, [C.c_int, C.POINTER(GemmDesc), C.POINTER(GemmDesc), C.c_void_p]
+    d = Dev(k)
+    try:
+        pg, pw, px = d.put(G), d.put(W), d.put(X)
+        cx, cw = d.put(np.zeros((M, K), np.float32)), d.put(np.zeros((K, N), np.float32))
+        dd = GemmDesc(M, K, N, pg, N, 0, M, pw, N, 0, K, cx, K, 0, 1, 0)
+        dwd = GemmDesc(K, N, M, px, K, 0, K, pg, N, 0, N, cw, N, 0, 1, 0)
+        assert fn(BF16, C.byref(dd), C.byref(dwd), k.pgd_stream()) == 0
+        pair = d.get(cx, (M, K), np.float32), d.get(cw, (K, N), np.float32)
+        for ta, x in ((0, dd), (1, dwd)):
+            wsz = k.pgk_gemm16_workspace_cu(ta, ta, x.m, x.n, x.k, 1, 255)
+            ws = d.put(np.zeros(max(wsz, 16), np.uint8))
+            assert k.pgk_gemm16_plan(ta, ta, x.m, x.n, x.k, 1, 255, None) < 5
+            assert k.pgk_gemm16_cu(BF16, ta, ta, x.m, x.n, x.k, x.a, x.lda, 0, x.a_extent, x.b, x.ldb, 0, x.b_extent,
+                                   x.c, x.ldc, 0, 1, 0, None, ws, 255, k.pgd_stream()) == 0
+        split = d.get(cx, (M, K), np.float32), d.get(cw, (K, N), np.float32)
+    finally:
+        d.free()
+    for name, got, ref, old in zip(("dX", "dW"), pair, refs, split):
+        e, eo = np.linalg.norm(got - ref), np.linalg.norm(old - ref)
+        assert e <= 1.05 * eo, (name, e / np.linalg.norm(ref), eo / np.linalg.norm(ref))
+
+
 @pytest.mark.parametrize("M,K,N", [(30, 1202, 10), (118, 2275, 11)])
 def test_matmul_with_small_grads(lib, oracle, M, K, N):
     """Grads that no one launch holds and that run one after the other."""
