@@ -1569,16 +1569,29 @@ static constexpr int kCUs = 256;
 
 // The split-over-waves tile for `problems` problems run as one launch, 0 when
 // none: the smallest tile whose blocks all run at once, one per CU (two for
-// the 64 x 64 tile).  Each beats the larger ones and the 128-tile plans up to
-// that count at every reduction measured (128 to 4096: 32 x 32 at 256 blocks
-// 3.7 - 13 against 7.2 - 20 us; 64 x 64 at 512 blocks 7.1 - 33 against 7.5 -
-// 36 us); past it they lose (64 x 64 at 1024 blocks 12 - 21 against 7.6 - 17
-// us).  A 64 x 64 tile takes eight waves in place of four for a long
-// reduction that leaves one block per CU: the same time (8.4 and 8.5 us at
-// 1024^3), and as many partial sums as the split-K plan there has, so the
-// error against 64 bits stays where it was (1.5e-7 at k = 4096, 1.9e-7 with
-// four).  Products of at most 16 columns keep their plans: more than half of
-// these tiles would be padding.
+// the 64 x 64 tile), up to the longest reduction at which it still wins.
+// Blocks: each tile beats the larger ones up to its count (32 x 32 at 256
+// blocks 3.7 - 13 against 7.2 - 20 us; 64 x 64 at 512 blocks 7.1 - 33 against
+// 7.5 - 36 us, k 128 to 2816) and loses past it (64 x 64 at 1024 blocks 12 - 21
+// against 7.6 - 17 us).
+// Reductions: a block's waves stream its operands through one CU where
+// split-K's eight slices have eight, so long ones are the split's (500 shapes,
+// other inputs in every launch).  Alone, a 32 x 32 tile is 1.0 - 2.4 times as
+// fast up to k = 6144 and slower from there (wgrad 72 x 1080 at 7520: 27 against
+// 23 us; 512 x 512 at 65536: 175 against 93), 32 x 64 to 4608 (72 x 3080 at 5272:
+// 29 against 22), both only to 2816 when the operands pass 18 MiB (45 x 3592 at
+// 3768: 24 against 19 us, 62 x 3584 at 2752: 10 against 17); 64 x 64 to 2816 with
+// two blocks on a CU (2232 x 528 at 2888: 29 against 24) and to 4096 with one
+// (360 x 1904 at 4608: 28 against 21; 2048 x 1024 at 65536: 659 against 236).
+// A pair saves launches too and holds further, 8192 for tiles of 32 rows (rows
+// 7080, 32 x 24: 10 us against 15 apart), 4096 and 7168 for 64 x 64: past it the
+// long wgrad is a few blocks of a tile larger than its own (8192 x 64 x 64:
+// 25 against 23 us, 16384 x 64 x 64: 55 against 32).
+// 64 x 64 tiles take eight waves in place of four for a long reduction that
+// leaves one block per CU: the same time (8.4 and 8.5 us at 1024^3), with a
+// shorter chain of sums per wave.  plan_gemm keeps products of at most 16
+// columns from these tiles (more than half would be padding); in a pair they
+// are welcome (rows 6928, 16 x 88: 16 us in one launch, 22 in two).
 struct ks_size {
     size_t m, n, batch, k;
 };
@@ -1586,16 +1599,22 @@ static int ks_tile(std::initializer_list<ks_size> problems)
 {
     static const struct {
         int tile;
-        size_t tm, tn, most;
-    } shapes[3] = {{5, 32, 32, 256}, {6, 32, 64, 256}, {7, 64, 64, 512}};
+        size_t tm, tn, most, k_alone, k_pair;
+    } shapes[4] = {{5, 32, 32, 256, 6144, 8192}, {6, 32, 64, 256, 4608, 8192}, {8, 64, 64, 256, 4096, 7168},
+                   {7, 64, 64, 512, 2816, 4096}};
+    const bool pair = problems.size() > 1;
     for (const auto &sh : shapes) {
-        size_t blocks = 0, k = 0;
+        size_t blocks = 0, k = 0, bytes = 0;
         for (const ks_size &q : problems) {
             blocks += ((q.m + sh.tm - 1) / sh.tm) * ((q.n + sh.tn - 1) / sh.tn) * q.batch;
             k = q.k > k ? q.k : k;
+            bytes += 2 * (q.m + q.n) * q.k * q.batch;
         }
-        if (blocks <= sh.most)
-            return sh.tile == 7 && blocks <= 256 && k >= 1024 ? 8 : sh.tile;
+        if (blocks > sh.most)
+            continue;
+        if (k > (pair ? sh.k_pair : sh.k_alone) || (!pair && sh.tm == 32 && k > 2816 && bytes > ((size_t)18 << 20)))
+            return 0;
+        return sh.tile == 8 && k < 1024 ? 7 : sh.tile;
     }
     return 0;
 }

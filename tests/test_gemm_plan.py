@@ -1,5 +1,7 @@
-"""The GEMM planner's choices, which need no device: which f32 grads
-share a launch, and when the two grads of a matmul may run on two streams."""
+"""The GEMM planner's choices, which need no device: which products take the
+tiles whose waves split the reduction (planner tiles 5 to 8), alone and as a
+dgrad + wgrad pair, which f32 grads share a launch, and when the two grads of
+a matmul may run on two streams."""
 from __future__ import annotations
 
 import ctypes as C
@@ -7,6 +9,7 @@ import ctypes as C
 import pytest
 
 import picograd_amd
+from test_gpu_gemm_guard import GemmDesc
 
 
 @pytest.fixture(scope="module")
@@ -14,8 +17,37 @@ def k():
     lib = picograd_amd.load().lib
     sz, i = C.c_size_t, C.c_int
     lib.pgk_gemm16_plan.restype, lib.pgk_gemm16_plan.argtypes = i, [i, i, sz, sz, sz, sz, i, C.POINTER(i)]
+    lib.pgk_gemm16_ks_pair_tile.restype = i
+    lib.pgk_gemm16_ks_pair_tile.argtypes = [C.POINTER(GemmDesc), C.POINTER(GemmDesc)]
     lib.pgm_grad_split.restype, lib.pgm_grad_split.argtypes = i, [sz] * 7 + [C.POINTER(C.c_bool)]
     return lib
+
+
+def pair_tile(k, M, K, N):
+    """For dX [M, K] = G W^T and dW [K, N] = X^T G."""
+    d = GemmDesc(M, K, N, 16, N, 0, M, 16, N, 0, K, 16, K, 0, 1, 0)
+    w = GemmDesc(K, N, M, 16, K, 0, K, 16, N, 0, N, 16, N, 0, 1, 0)
+    return k.pgk_gemm16_ks_pair_tile(C.byref(d), C.byref(w))
+
+
+@pytest.mark.parametrize("m,n,kk,tile", [
+    (512, 512, 4096, 5), (512, 512, 65536, 0), (64, 64, 16384, 0), (72, 1080, 7520, 0),
+    (512, 1024, 4096, 6), (512, 1024, 16384, 0), (1024, 1024, 4096, 8), (1024, 1024, 16384, 0),
+    (2048, 1024, 2048, 7), (2048, 1024, 12288, 0), (440, 3440, 5080, 0), (2232, 528, 2888, 0), (45, 3592, 3768, 0),
+])
+def test_long_reductions_keep_the_split_over_blocks(k, m, n, kk, tile):
+    """A tile of one CU is taken up to the reduction at which eight slices of
+    the chip are faster; 0 here is any of the tiled plans."""
+    got = k.pgk_gemm16_plan(1, 1, m, n, kk, 1, 0, None)
+    assert got == tile if tile else got in (1, 2, 3)
+
+
+@pytest.mark.parametrize("M,K,N,tile", [
+    (8192, 128, 1024, 0), (16384, 64, 512, 0), (16384, 64, 2048, 0), (8192, 64, 64, 0), (16384, 64, 64, 0),
+    (4096, 64, 1024, 6), (4096, 256, 2048, 7), (7080, 32, 24, 5), (6928, 16, 88, 5), (5056, 80, 32, 8),
+])
+def test_pairs_look_at_the_longer_reduction(k, M, K, N, tile):
+    assert pair_tile(k, M, K, N) == tile
 
 
 @pytest.mark.parametrize("m,kk,n,tile", [(8192, 64, 64, 0), (16384, 64, 64, 0), (2048, 256, 256, 0), (752, 424, 66, 0),

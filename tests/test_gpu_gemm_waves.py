@@ -87,7 +87,8 @@ def test_few_rows(lib, oracle, k, m, n, kk, beta, dt):  # noqa: F811
 
 
 @pytest.mark.parametrize("dt", [BF16, F16])
-@pytest.mark.parametrize("shape", [(40, 72, 104), (257, 264, 520), (130, 512, 1024), (1030, 264, 520), (500, 1000, 520), (96, 208, 616)],
+@pytest.mark.parametrize("shape", [(40, 72, 104), (257, 264, 520), (130, 512, 1024), (1030, 264, 520), (500, 1000, 520), (96, 208, 616),
+                                   (8160, 24, 32), (32, 32, 8192), (7160, 72, 72), (4096, 256, 200)],
                          ids=lambda s: "%dx%dx%d" % s)
 def test_pair_in_one_launch(lib, oracle, k, shape, dt):  # noqa: F811
     """dX = G.W^T and dW = X^T.G of C = X.W, X [M, K], W [K, N]; dW accumulates."""
