@@ -1696,10 +1696,15 @@ static bool skinny_ok(int ta, int tb, size_t m, size_t n, size_t k, size_t batch
 
 // k_few_rows's products: one 16-row tile with a block per CU at most (past
 // 4096 columns the wider tiles stream faster: 22.5 against 37.5 us at 11008),
-// or a few such tiles of one column tile
+// or a few such tiles of one column tile.  Reductions as above: up to 4096 it
+// is the faster one at every width, up to 12288 while B has at most 12 Mi
+// elements (1088 columns at 8080: 17 against 18 us; 3232 at 6192: 23 against
+// 18, 64 at 18896: 31 against 23), and up to 32768 for one column tile (8 at
+// 33296: 24 against 34 us).
 static bool few_rows_ok(int ta, int tb, size_t m, size_t n, size_t k, size_t batch)
 {
-    return !ta && tb && batch == 1 && k && k % 8 == 0 && ((m <= 16 && n <= 4096) || (m <= 64 && n <= 16));
+    return !ta && tb && batch == 1 && k && k % 8 == 0 && ((m <= 16 && n <= 4096) || (m <= 64 && n <= 16)) &&
+           (k <= 4096 || (k <= 12288 && n * k <= (size_t)12 << 20) || (k <= 32768 && n <= 16));
 }
 
 static size_t tail_ws(int ta, int tb, size_t m, size_t n, size_t k, size_t batch)

@@ -1,7 +1,7 @@
 """The GEMM planner's choices, which need no device: which products take the
-tiles whose waves split the reduction (planner tiles 5 to 8), alone and as a
-dgrad + wgrad pair, which f32 grads share a launch, and when the two grads of
-a matmul may run on two streams."""
+tiles whose waves split the reduction (planner tiles 5 to 8) and the few-rows
+kernel (9), alone and as a dgrad + wgrad pair, which f32 grads share a launch,
+and when the two grads of a matmul may run on two streams."""
 from __future__ import annotations
 
 import ctypes as C
@@ -40,6 +40,12 @@ def test_long_reductions_keep_the_split_over_blocks(k, m, n, kk, tile):
     the chip are faster; 0 here is any of the tiled plans."""
     got = k.pgk_gemm16_plan(1, 1, m, n, kk, 1, 0, None)
     assert got == tile if tile else got in (1, 2, 3)
+
+
+@pytest.mark.parametrize("m,n,kk,few", [(16, 4096, 4096, True), (16, 128, 8192, True), (64, 16, 32768, True),
+                                        (5, 3232, 6192, False), (13, 64, 18896, False), (16, 3376, 25800, False)])
+def test_few_rows_up_to_the_measured_reductions(k, m, n, kk, few):
+    assert (k.pgk_gemm16_plan(0, 1, m, n, kk, 1, 0, None) == 9) == few
 
 
 @pytest.mark.parametrize("M,K,N,tile", [
