@@ -1848,6 +1848,8 @@ extern "C" int pgk_gemm16_cu(int dtype, int ta, int tb, size_t m, size_t n, size
     // the epilogue rides on the GEMM when one launch of the forward layout
     // finishes C, on the split-K sum when that finishes C, otherwise it is
     // a pass over C afterwards
+    if ((sp || ktail) && !ws)
+        return (int)hipErrorInvalidValue;
     if (pl.tile >= 5 && kmain) {
         const bool fused = has_epi && !ktail;
         gemm_args g = {a, lda, stride_a, (int)a_extent, b, ldb, stride_b, (int)b_extent, c, ldc, stride_c,
@@ -1862,8 +1864,6 @@ extern "C" int pgk_gemm16_cu(int dtype, int ta, int tb, size_t m, size_t n, size
                    : launch_layout<false, true, false, true>(g, st, *epi);
     }
     const size_t part_bytes = sp ? (((size_t)sp * m * n * sizeof(float) + 255) & ~(size_t)255) : 0;
-    if ((sp || ktail) && !ws)
-        return (int)hipErrorInvalidValue;
     int rc = 0;
     if (pl.tile >= 5) {
         // queued above; a k tail and its epilogue follow

@@ -160,6 +160,23 @@ def test_pair_error_is_no_larger_than_the_split(lib, oracle, k, M, K, N):
         assert e <= 1.05 * eo, (name, e / np.linalg.norm(ref), eo / np.linalg.norm(ref))
 
 
+def test_missing_workspace_is_refused_before_anything_is_queued(lib, oracle, k):
+    """A reduction with a tail (k % 8) on a tile of this file needs a workspace."""
+    m, n, kk = 40, 48, 77
+    rng = np.random.default_rng(1)
+    A, B = (oracle.cast16(BF16, rng.standard_normal(s).astype(np.float32)) for s in ((m, 80), (n, 80)))
+    c0 = rng.standard_normal((m, n)).astype(np.float32)
+    assert k.pgk_gemm16_plan(0, 0, m, n, kk, 1, 0, None) == 5 and k.pgk_gemm16_workspace_cu(0, 0, m, n, kk, 1, 0)
+    d = Dev(k)
+    try:
+        pa, pb, pc = d.put(A), d.put(B), d.put(c0)
+        assert k.pgk_gemm16_cu(BF16, 0, 0, m, n, kk, pa, 80, 0, m, pb, 80, 0, n, pc, n, 0, 1, 0, None, None, 0,
+                               k.pgd_stream()) != 0
+        assert np.array_equal(d.get(pc, c0.shape, np.float32), c0)
+    finally:
+        d.free()
+
+
 @pytest.mark.parametrize("M,K,N", [(30, 1202, 10), (118, 2275, 11)])
 def test_matmul_with_small_grads(lib, oracle, M, K, N):
     """Grads that no one launch holds and that run one after the other."""
