@@ -113,6 +113,10 @@ __device__ __forceinline__ void dma16s(uint32_t voff, const void *sbase, LDS uin
 // end of the reduction dim, so a partial last k-tile lands zero-filled
 __device__ const uint4 g_zero16 = {0u, 0u, 0u, 0u};
 
+// leading dims under this take the fast loads below: their 32-bit lane
+// offsets span at most 16 rows
+constexpr size_t kFastLd = (size_t)1 << 26;
+
 // K-contiguous operand tile: ROWS x KB (KB = 64 or 32), rows of KB / 8
 // 16-byte chunks.  Load instruction q of wave w fills chunk slots
 // (w NQ + q) 64 .. + 63.  Chunks are XOR-swizzled within a row so the 16
@@ -151,7 +155,7 @@ struct TileK {
     // `srow` (the first row load q touches, clamped like the rows) and each
     // lane's offset is (its clamped row - srow) ld + its chunk, in bytes;
     // the 64 lanes span 64 / CH rows, so the offset fits 32 bits for
-    // ld < 2^26.  `wave` must be wave-uniform.
+    // ld < kFastLd.  `wave` must be wave-uniform.
     struct Fast {
         uint32_t voff;
         int srow;
@@ -221,7 +225,10 @@ struct TileMN {
     // Fast form of load q (k-tiles below kend): the scalar base is k-row
     // k0 + kq (the first k-row load q touches), column row0, and each lane's
     // offset is (its k-row - kq) ld + (its clamped column - row0), in bytes;
-    // the 64 lanes span 64 / CPR <= 4 k-rows.  `wave` must be wave-uniform.
+    // the 64 lanes span 64 / CPR k-rows, at most 16, so leading dims under
+    // kFastLd keep it within 32 bits.  `wave` must be wave-uniform.
+    static_assert((uint64_t)(64 / CPR > 1 ? 64 / CPR - 1 : 1) * kFastLd * 2 + ROWS * 2 < ((uint64_t)1 << 32),
+                  "a load's lane offsets fit 32 bits");
     struct Fast {
         uint32_t voff;
         int srow;
@@ -383,7 +390,7 @@ __device__ __forceinline__ void gemm16_block(const gemm_kargs &g, int pid, int n
             OB::load_q(q - OA::NQ, Bb, ldb, n0, b_extent, t * KB, kend, dB, tid);
     };
     // per-lane offsets of the fast form (tiles wholly below kend, leading
-    // dims under 2^26: fast_ok), fixed for the whole k-loop
+    // dims under kFastLd: fast_ok), fixed for the whole k-loop
     typename OA::Fast fA[OA::NQ];
     typename OB::Fast fB[OB::NQ];
 #pragma unroll
@@ -1301,7 +1308,7 @@ gemm_kargs make_kargs(const gemm_args &g, const pgk_epi &epi)
     k.tiles_m = (g.m + CF::BM - 1) / CF::BM, k.tiles_n = (g.n + CF::BN - 1) / CF::BN;
     k.epi = epi;
     k.k_total = g.k_total ? g.k_total : g.k, k.kz_step = g.kz_step;
-    k.fast_ok = (int)(g.lda < ((size_t)1 << 26) && g.ldb < ((size_t)1 << 26));
+    k.fast_ok = (int)(g.lda < kFastLd && g.ldb < kFastLd);
     return k;
 }
 
