@@ -149,7 +149,7 @@ def test_grads_summed_over_other_dims_stay_apart(lib):
 
 
 def test_grads_accumulate_into_existing_ones(lib):
-    """x feeds the run and a second branch: the region adds to x's grad (beta 1)."""
+    """x feeds the run and a product below it, whose grad adds to the one the region wrote."""
     rng = np.random.default_rng(6)
     x = rng.standard_normal((260, 68)).astype(np.float32)
     got = {}
@@ -170,3 +170,37 @@ def test_grads_accumulate_into_existing_ones(lib):
             lib.pg_autograd_set_jit(True)
     for a, b in zip(got[True], got[False]):
         assert np.abs(a - b).max() <= 5e-6 * max(1.0, np.abs(b).max())
+
+
+@pytest.mark.parametrize("cols", [68, 1037, 128])
+def test_region_adds_to_an_existing_grad(lib, cols):
+    """loss = sum(tanh(x + b) @ w1 + x @ w2): the walk reaches x @ w2 first, so the
+    region of tanh and + adds to x's grad (beta 1) beside the bias grad it sums.
+    Columns: whole 16-byte pieces that end inside a 128-byte line, odd, and whole
+    lines."""
+    rng = np.random.default_rng(cols)
+    rows, n = 300, 24
+    x = rng.standard_normal((rows, cols)).astype(np.float32)
+    b = (0.1 * rng.standard_normal(cols)).astype(np.float32)
+    w1, w2 = ((cols ** -0.5 * rng.standard_normal((cols, n))).astype(np.float32) for _ in range(2))
+    nx, nb, n1, n2 = lib.var(x), lib.var(b), lib.var(w1), lib.var(w2)
+    made = [lib.op("add", nx, nb)]
+    made.append(lib.op("tanh", made[-1]))
+    m1 = lib.op("matmul", made[-1], n1)
+    m2 = lib.op("matmul", nx, n2)
+    y = lib.op("add", m1, m2)
+    loss = lib.op("sum_all", y)
+    lib.pg_backward(loss)
+    assert lib.pg_autograd_last_was_jit(), lib.pg_autograd_last_error().decode()
+    x64, b64, w1d, w2d = (v.astype(np.float64) for v in (x, b, w1, w2))
+    t = np.tanh(x64 + b64)
+    dt = (1 - t * t) * w1d.sum(1)
+    ref = {"dx": dt + w2d.sum(1), "db": dt.sum(0), "dw1": np.repeat(t.sum(0)[:, None], n, 1)}
+    # products of 24 terms, tanh and its grad to a few units in the last place, then rows + 16 additions for db
+    u = 2.0 ** -24
+    mag = np.abs(w1d).sum(1) + np.abs(w2d).sum(1)
+    assert (np.abs(lib.grad(nx) - ref["dx"]) <= 64 * u * mag).all()
+    assert (np.abs(lib.grad(nb) - ref["db"]) <= (rows + 64) * u * rows * np.abs(w1d).sum(1)).all()
+    assert (np.abs(lib.grad(n1) - ref["dw1"]) <= (rows + 64) * u * np.abs(t).sum(0)[:, None]).all()
+    for v in (loss, y, m2, m1, *reversed(made), n2, n1, nb, nx):
+        lib.pg_node_free(v)
