@@ -477,8 +477,8 @@ static bool run_region(wctx *w, int r, const pg_tensor *root_grad, float scale, 
         }
     }
     if (ok) {
-        /* a small forward run still pending (config 1: leaves, forward and
-         * sum in one block) takes the region into its own launch */
+        /* a forward run still pending takes the region into its own launch
+         * (a small one into its one block: config 1's leaves, forward and sum) */
         ok = pga_lazy_flush_with_backward(b.g, L->ndim, L->shape, b.in_ptr, b.nin, optr, nout + n16) ||
              pgj_launch(b.g, L->ndim, L->shape, b.in_ptr, b.nin, optr, nout + n16);
         for (size_t i = 0; ok && i < n16; i++)
