@@ -147,8 +147,9 @@ size_t pg_amd_jit_cache_hits(void);
  * kernel for n <= 16 with B MN-contiguous and at least 1009 rows, 16 rows
  * of C per block, one launch with no split; 5 to 8: tiles of 32 x 32,
  * 32 x 64 and 64 x 64 (two forms) whose waves split the reduction, for outputs that
- * 128-tiles would not spread over the chip; 9: the few-rows kernel, 16 x 16
- * tiles for m <= 16), stores the
+ * 128-tiles would not spread over the chip, up to a reduction of a few
+ * thousand; 9: the few-rows kernel, 16 x 16 tiles for m <= 16, or m <= 64 with
+ * n <= 16), stores the
  * split-K factor (1 = none) in *splits and the planner's time estimate in
  * seconds in *seconds (either may be NULL).  cu_budget: the CUs the launch
  * may occupy when it shares the chip with another (a matmul's dgrad and

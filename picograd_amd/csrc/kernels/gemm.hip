@@ -1013,10 +1013,10 @@ __global__ void __launch_bounds__(C1::NT, C1::KG == 4 ? 2 : 1) k_gemm16_ks_pair(
 // reduction as k_gemm16_ks's do, each with a three-stage ring of 64-deep
 // chunks of its own.  Tiles of 16 x 16 (v_mfma_f32_16x16x32) halve what A costs
 // the 32-row ones.  Bound by the stream of 32-byte row pieces: 16 x 4096 x 4096
-// takes 11.7 us (2.9 TB/s; 64-column pieces would take 8.8 without the sum
-// across blocks that they need), against 14.3 on 32 x 32 tiles and 19 for
-// split-K and its sum; 16 x 10 x 4096 takes 4.6 us against 10.8.  Two or four
-// stages, sixteen waves and 32 columns a block measured the same or slower.
+// takes 11.4 us back to back (2.9 TB/s; 10.8 in the kernel, 3.1; 64-column
+// pieces would take 8.8 without the sum across blocks that they need), against
+// 14.3 on 32 x 32 tiles and 18.3 for split-K and its sum; 16 columns of the
+// same take 5.9 us against 12.9.  Two or four stages, sixteen waves and 32 columns a block measured the same or slower.
 typedef float f32x4m __attribute__((ext_vector_type(4)));
 
 template <bool F16>
