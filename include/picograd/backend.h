@@ -33,8 +33,10 @@ void pg_bgemm(size_t m, size_t n, size_t k, const uint16_t *a, size_t lda, const
  * contract, kernels and result bits as pg_gemm_ex; the buffers those need
  * (zero-padded operand copies, split-K partials, k-tail slabs) come from a
  * fixed 32 MiB workspace that each device holds for the life of the
- * process, instead of the library allocator.  A call whose buffers exceed
- * it is rejected.  Calls share the workspace: they are ordered on the
+ * process, instead of the library allocator.  A product whose split-K
+ * partials alone exceed it runs on a tile that needs none where there is one
+ * (its sums are then in another order than pg_gemm_ex's).  Any other call whose
+ * buffers exceed it is rejected.  Calls share the workspace: they are ordered on the
  * library stream, and calls overlapping on one device from two host
  * threads would race.  Work other calls left waiting to be queued (batched
  * uploads, deferred elementwise ops: queueing them may compile, allocate or

@@ -537,7 +537,9 @@ int pg_amd_gemm16_plan(int ta, int tb, size_t m, size_t n, size_t k, size_t batc
  * instead of the library allocator.  The operands take the same path as in
  * pg_gemm_ex (read in place when the leading dims and bases allow 16-byte
  * loads and n is a multiple of 8, else both padded to [m, K8] and [K8, N8]),
- * so the kernels, the launch plan and the result bits are the same. */
+ * so the kernels, the launch plan and the result bits are the same -- but for
+ * a product whose split-K partials alone do not fit, which runs on a tile that
+ * needs none where there is one (its sums in another order). */
 static size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 int pg_amd_gemm_ex_noalloc(pg_dtype dtype, size_t m, size_t n, size_t k, const void *a, size_t lda, const void *b,
@@ -580,7 +582,8 @@ int pg_amd_gemm_ex_noalloc(pg_dtype dtype, size_t m, size_t n, size_t k, const v
     size_t K8 = direct ? k : up8(k), N8 = up8(n) < 8 ? 8 : up8(n);
     size_t abytes = direct ? 0 : up256(m * K8 * 2), bbytes = direct ? 0 : up256(K8 * N8 * 2);
     size_t wsz = pgk_gemm16_workspace(0, 1, m, n, K8, 1);
-    size_t need = abytes + bbytes + wsz;
+    const bool lean = abytes + bbytes + wsz > cap && pgk_gemm16_lean_tile(0, 1, m, n, K8, 1);
+    size_t need = abytes + bbytes + (lean ? 0 : wsz);
     if (need > cap) {
         pgd_set_err("pg_amd_gemm_ex_noalloc: %zux%zux%zu needs %zu bytes of workspace, above the no-alloc "
                     "maximum of %zu",
@@ -599,8 +602,9 @@ int pg_amd_gemm_ex_noalloc(pg_dtype dtype, size_t m, size_t n, size_t k, const v
         lda2 = K8;
         ldb2 = bext = N8;
     }
-    int rc = pgk_gemm16(dt, 0, 1, m, n, K8, ap, lda2, 0, m, bp, ldb2, 0, bext, c, ldc, 0, 1, 0, NULL,
-                        wsz ? ws + abytes + bbytes : NULL, st);
+    int rc = lean ? pgk_gemm16_lean(dt, 0, 1, m, n, K8, ap, lda2, 0, m, bp, ldb2, 0, bext, c, ldc, 0, 1, 0, st)
+                  : pgk_gemm16(dt, 0, 1, m, n, K8, ap, lda2, 0, m, bp, ldb2, 0, bext, c, ldc, 0, 1, 0, NULL,
+                               wsz ? ws + abytes + bbytes : NULL, st);
     return pgd_check(rc, "pg_amd_gemm_ex_noalloc") ? 0 : -1;
 }
 

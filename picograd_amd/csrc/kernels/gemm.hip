@@ -1602,7 +1602,7 @@ static constexpr int kCUs = 256;
 struct ks_size {
     size_t m, n, batch, k;
 };
-static int ks_tile(std::initializer_list<ks_size> problems)
+static int ks_tile(std::initializer_list<ks_size> problems, bool any_k = false)
 {
     static const struct {
         int tile;
@@ -1619,6 +1619,8 @@ static int ks_tile(std::initializer_list<ks_size> problems)
         }
         if (blocks > sh.most)
             continue;
+        if (any_k)
+            return sh.tile == 8 && k < 1024 ? 7 : sh.tile;
         if (k > (pair ? sh.k_pair : sh.k_alone) || (!pair && sh.tm == 32 && k > 2816 && bytes > ((size_t)18 << 20)))
             return 0;
         return sh.tile == 8 && k < 1024 ? 7 : sh.tile;
@@ -1928,6 +1930,27 @@ extern "C" int pgk_gemm16_cu(int dtype, int ta, int tb, size_t m, size_t n, size
         return (int)hipGetLastError();
     }
     return 0;
+}
+
+// Without a workspace: the split-over-waves tile by its block count alone, for
+// a caller whose fixed workspace cannot hold the faster plan's partials
+extern "C" int pgk_gemm16_lean_tile(int ta, int tb, size_t m, size_t n, size_t k, size_t batch)
+{
+    return m && n && batch && k && k_inkernel(ta, tb, k) == k ? ks_tile({{m, n, batch, k}}, true) : 0;
+}
+
+extern "C" int pgk_gemm16_lean(int dtype, int ta, int tb, size_t m, size_t n, size_t k, const uint16_t *a, size_t lda,
+                               size_t stride_a, size_t a_extent, const uint16_t *b, size_t ldb, size_t stride_b,
+                               size_t b_extent, float *c, size_t ldc, size_t stride_c, size_t batch, int beta,
+                               pgk_stream s)
+{
+    const int tile = pgk_gemm16_lean_tile(ta, tb, m, n, k, batch);
+    const int bad = check_gemm_args(ta, tb, m, n, k, a, lda, stride_a, a_extent, b, ldb, stride_b, b_extent, batch);
+    if (!tile || bad)
+        return bad ? bad : (int)hipErrorInvalidValue;
+    const gemm_args g = {a, lda, stride_a, (int)a_extent, b, ldb, stride_b, (int)b_extent, c, ldc, stride_c,
+                         (int)m, (int)n, (int)k, beta, (unsigned)batch, tile};
+    return launch_ks_any(dtype == 1, ta, tb, g, pgk_epi{}, 0, (hipStream_t)s);
 }
 
 extern "C" size_t pgk_gemm16_pair_dw_workspace(const pgk_gemm_desc *d, const pgk_gemm_desc *w, int cu_d, size_t *off_w)

@@ -168,6 +168,13 @@ int pgk_gemm16_cu(int dtype, int ta, int tb, size_t m, size_t n, size_t k, const
                   int cu_budget, pgk_stream s);
 size_t pgk_gemm16_workspace_cu(int ta, int tb, size_t m, size_t n, size_t k, size_t batch, int cu_budget);
 double pgk_gemm16_time(int ta, int tb, size_t m, size_t n, size_t k, size_t batch, int cu_budget);
+/* C (beta ? += : =) A B without any workspace, on the split-over-waves tile of
+ * its block count whatever its reduction; _tile is that tile, 0 when there is
+ * none (the launch is then refused). */
+int pgk_gemm16_lean_tile(int ta, int tb, size_t m, size_t n, size_t k, size_t batch);
+int pgk_gemm16_lean(int dtype, int ta, int tb, size_t m, size_t n, size_t k, const uint16_t *a, size_t lda,
+                    size_t stride_a, size_t a_extent, const uint16_t *b, size_t ldb, size_t stride_b, size_t b_extent,
+                    float *c, size_t ldc, size_t stride_c, size_t batch, int beta, pgk_stream s);
 /* the tile (1: 128 x 128, 2: 256 x 256, 3: 128 x 256) and split-K factor
  * (*splits) pgk_gemm16_cu's main launch takes for these sizes */
 int pgk_gemm16_plan(int ta, int tb, size_t m, size_t n, size_t k, size_t batch, int cu_budget, int *splits);

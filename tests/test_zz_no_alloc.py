@@ -6,14 +6,16 @@ same bits.  Two calls in a row, the second with a smaller input (the
 workspace keeps the first call's contents), each checked against
 pg_gemm_ex and against the f32-accumulating oracle; the library's allocator
 must see no allocation during the calls; a GEMM whose split-K partials need
-more than the workspace is refused with an error and leaves C untouched.
+more than the workspace runs without them where a tile allows it, and is else
+refused with an error and leaves C untouched.
 """
 import ctypes as C
 
 import numpy as np
 import pytest
 
-from oracle_lib import rel_fro
+from gemm_check import check_product
+from oracle_lib import bf16_to_f32, f16_to_f32, rel_fro
 from picograd_amd.capi import BF16, F16, F32
 
 pytestmark = pytest.mark.gpu
@@ -97,6 +99,31 @@ def test_noalloc_gemm_other_shapes(lib, oracle, dt, m, n, k):
     got, want = lib.read(cs.c_new), lib.read(cs.c_ref)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
     assert rel_fro(got, oracle.gemm(dt, cs.a16, cs.b16)) <= 1e-5
+    cs.free(lib)
+
+
+@pytest.mark.parametrize("dt,m,n,k", [(F16, 407, 1664, 5145), (BF16, 42, 2316, 6807), (BF16, 2752, 576, 6656)])
+def test_noalloc_gemm_without_room_for_partials(lib, oracle, dt, m, n, k):
+    """Operand copies (or none) that fit the workspace, with split-K partials that do not
+    fit behind them: a tile without partials, accepted and right.  (Reductions under
+    about 10000: past that gamma(K) sum|AB| nears the size of a typical element, and
+    check_product's own planted mistakes pass the bound.)"""
+    cap = 32 << 20
+    up = lambda x, a: -(-x // a) * a  # noqa: E731
+    k8, n8 = up(k, 8), up(n, 8)
+    copies = 0 if (n8, k8) == (n, k) else up(m * k8 * 2, 256) + up(k8 * n8 * 2, 256)
+    ws = lib.lib.pgk_gemm16_workspace
+    ws.restype, ws.argtypes = C.c_size_t, [C.c_int, C.c_int] + [C.c_size_t] * 4
+    assert copies <= cap < copies + ws(0, 1, m, n, k8, 1), "the planner no longer splits this shape"
+    print(f"no-alloc gemm without partials dt={dt} m={m} n={n} k={k}", flush=True)
+    cs = _Case(lib, oracle, dt, m, n, k, m)
+    lib.sync()
+    used, cached = lib.pg_amd_bytes_in_use(), lib.pg_amd_bytes_cached()
+    assert cs.run_new(lib) == 0, lib.pg_amd_last_error().decode()
+    lib.sync()
+    assert (lib.pg_amd_bytes_in_use(), lib.pg_amd_bytes_cached()) == (used, cached)
+    f32 = f16_to_f32 if dt == F16 else bf16_to_f32
+    check_product(lib.read(cs.c_new), [(f32(cs.a16), f32(cs.b16))], "no-alloc gemm without partials")
     cs.free(lib)
 
 
