@@ -814,6 +814,15 @@ struct kscfg {
     static constexpr int LDS_U4 = RING > PART ? RING : PART;
 };
 
+// block id -> tile: ids are dealt to the 8 XCDs round-robin (from any first
+// one), so consecutive tiles, which share lines and panels of the operands, are
+// regrouped onto one XCD and its L2; the last nb % 8 stay where they are
+__device__ __forceinline__ int xcd_tile(int pid, int nb)
+{
+    const int q = nb >> 3;
+    return pid < (q << 3) ? (pid & 7) * q + (pid >> 3) : pid;
+}
+
 template <class CF>
 __device__ __forceinline__ void ks_block(const gemm_kargs &g, int has_epi, int pid, int nb, bool remap, int z,
                                          LDS uint4 *const lds)
@@ -827,9 +836,12 @@ __device__ __forceinline__ void ks_block(const gemm_kargs &g, int has_epi, int p
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     // tile order as the tiled kernel's: consecutive tiles on one XCD, 8
-    // tile-rows at a time
-    if (remap && (nb & 7) == 0)
-        pid = (pid & 7) * (nb >> 3) + (pid >> 3);
+    // tile-rows at a time.  Also for counts that 8 does not divide where the
+    // output is wider than tall: as dealt, every XCD fetches each line of the
+    // wide operand (98 x 3720 at k = 3008, 236 blocks: 26 us as dealt, 14
+    // grouped; 51 such shapes 0.99 - 1.7 times as fast, 95 tall ones 0.75 - 1.2)
+    if (g.tiles_n > g.tiles_m || (remap && (nb & 7) == 0))
+        pid = xcd_tile(pid, nb);
     const int group = pid / (8 * g.tiles_n), first = group * 8;
     const int gsz = g.tiles_m - first < 8 ? g.tiles_m - first : 8, in = pid - group * 8 * g.tiles_n;
     const int m0 = (first + in % gsz) * TM, n0 = in / gsz * TN;
@@ -1040,10 +1052,8 @@ __global__ void __launch_bounds__(kFrWaves * 64, 1) k_few_rows(gemm_kargs g, int
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     // neighbouring column tiles share each 128-byte line of a row: on one XCD
-    int pid = (int)blockIdx.x;
-    const int nb = (int)gridDim.x;
-    if ((nb & 7) == 0)
-        pid = (pid & 7) * (nb >> 3) + (pid >> 3);
+    // (9 x 4032 at k = 7232, 252 blocks: 33 us as dealt, 15 grouped)
+    const int pid = xcd_tile((int)blockIdx.x, (int)gridDim.x);
     const int n0 = pid * kFrTile, m0 = (int)blockIdx.y * kFrTile;
     LDS uint4 *const ring = (LDS uint4 *)smem + wave * kFrStages * (kFrA + kFrB);
     using TK = TileK<kFrTile, 64, kFrK>;
@@ -1582,18 +1592,17 @@ static constexpr int kCUs = 256;
 // 7.5 - 36 us, k 128 to 2816) and loses past it (64 x 64 at 1024 blocks 12 - 21
 // against 7.6 - 17 us).
 // Reductions: a block's waves stream its operands through one CU where
-// split-K's eight slices have eight, so long ones are the split's (500 shapes,
-// other inputs in every launch).  Alone, a 32 x 32 tile is 1.0 - 2.4 times as
-// fast up to k = 6144 and slower from there (wgrad 72 x 1080 at 7520: 27 against
-// 23 us; 512 x 512 at 65536: 175 against 93), 32 x 64 to 4608 (72 x 3080 at 5272:
-// 29 against 22), both only to 2816 when the operands pass 18 MiB (45 x 3592 at
-// 3768: 24 against 19 us, 62 x 3584 at 2752: 10 against 17); 64 x 64 to 2816 with
-// two blocks on a CU (2232 x 528 at 2888: 29 against 24) and to 4096 with one
-// (360 x 1904 at 4608: 28 against 21; 2048 x 1024 at 65536: 659 against 236).
-// A pair saves launches too and holds further, 8192 for tiles of 32 rows (rows
-// 7080, 32 x 24: 10 us against 15 apart), 4096 and 7168 for 64 x 64: past it the
-// long wgrad is a few blocks of a tile larger than its own (8192 x 64 x 64:
-// 25 against 23 us, 16384 x 64 x 64: 55 against 32).
+// split-K's eight slices have eight, so long ones are the split's (700 shapes,
+// other inputs in every launch).  Alone, a 32 x 32 tile is 0.95 - 2.5 times as
+// fast up to k = 10240 and with both operands MN-contiguous, whose every k row
+// is a 64-byte piece, 0.92 - 2 times up to 6144 (0.67 - 1 from 8192; 512 x 512 at
+// 65536: 175 against 93 us), 32 x 64 to 5632 (0.77 - 0.99 from 6144), 64 x 64 to
+// 4608 with one block on a CU and to 2816 with two (0.73 - 1.1 at 2816 - 4096;
+// 2048 x 1024 at 65536: 659 against 236 us).  A pair saves launches too and holds
+// to 8192 on tiles of 32 rows (1.2 - 2.4 times the two apart), on 64 x 64 to 7168
+// with one block on a CU and to 4096 with two: past it the long wgrad is a few
+// blocks of a tile larger than its own (f16 matmul with grads of 8192 x 128 x
+// 1024 52 against 43 us, 16384 x 64 x 64 65 against 39).
 // 64 x 64 tiles take eight waves in place of four for a long reduction that
 // leaves one block per CU: the same time (8.4 and 8.5 us at 1024^3), with a
 // shorter chain of sums per wave.  plan_gemm keeps products of at most 16
@@ -1602,26 +1611,22 @@ static constexpr int kCUs = 256;
 struct ks_size {
     size_t m, n, batch, k;
 };
-static int ks_tile(std::initializer_list<ks_size> problems, bool any_k = false)
+static int ks_tile(std::initializer_list<ks_size> problems, bool mn, bool any_k = false)
 {
     static const struct {
         int tile;
-        size_t tm, tn, most, k_alone, k_pair;
-    } shapes[4] = {{5, 32, 32, 256, 6144, 8192}, {6, 32, 64, 256, 4608, 8192}, {8, 64, 64, 256, 4096, 7168},
-                   {7, 64, 64, 512, 2816, 4096}};
-    const bool pair = problems.size() > 1;
+        size_t tm, tn, most, k_most, k_mn, k_pair; // k_mn: both operands MN-contiguous
+    } shapes[4] = {{5, 32, 32, 256, 10240, 6144, 8192}, {6, 32, 64, 256, 5632, 5632, 8192},
+                   {8, 64, 64, 256, 4608, 4608, 7168}, {7, 64, 64, 512, 2816, 2816, 4096}};
     for (const auto &sh : shapes) {
-        size_t blocks = 0, k = 0, bytes = 0;
+        size_t blocks = 0, k = 0;
         for (const ks_size &q : problems) {
             blocks += ((q.m + sh.tm - 1) / sh.tm) * ((q.n + sh.tn - 1) / sh.tn) * q.batch;
             k = q.k > k ? q.k : k;
-            bytes += 2 * (q.m + q.n) * q.k * q.batch;
         }
         if (blocks > sh.most)
             continue;
-        if (any_k)
-            return sh.tile == 8 && k < 1024 ? 7 : sh.tile;
-        if (k > (pair ? sh.k_pair : sh.k_alone) || (!pair && sh.tm == 32 && k > 2816 && bytes > ((size_t)18 << 20)))
+        if (!any_k && k > (problems.size() > 1 ? sh.k_pair : mn ? sh.k_mn : sh.k_most))
             return 0;
         return sh.tile == 8 && k < 1024 ? 7 : sh.tile;
     }
@@ -1646,11 +1651,12 @@ static double ks_time(int tile, size_t m, size_t n, size_t k, size_t batch)
 // reads sp and writes one, at ~5 TB/s, and one more launch.  A split must
 // still win by 8 % over the best plan without one: its partials also cost
 // HBM capacity.
-static gemm_plan plan_gemm(size_t m, size_t n, size_t kin, size_t batch, int cu_budget = 0, double *time = nullptr)
+static gemm_plan plan_gemm(int ta, int tb, size_t m, size_t n, size_t kin, size_t batch, int cu_budget = 0,
+                           double *time = nullptr)
 {
     const bool whole = !(cu_budget > 0 && cu_budget < kCUs);
     const double cus = whole ? (double)kCUs : (double)cu_budget;
-    const int ks = whole && n > 16 && kin ? ks_tile({{m, n, batch, kin}}) : 0;
+    const int ks = whole && n > 16 && kin ? ks_tile({{m, n, batch, kin}}, ta && tb) : 0;
     if (ks) {
         if (time)
             *time = ks_time(ks, m, n, kin, batch);
@@ -1705,15 +1711,13 @@ static bool skinny_ok(int ta, int tb, size_t m, size_t n, size_t k, size_t batch
 
 // k_few_rows's products: one 16-row tile with a block per CU at most (past
 // 4096 columns the wider tiles stream faster: 22.5 against 37.5 us at 11008),
-// or a few such tiles of one column tile.  Reductions as above: up to 4096 it
-// is the faster one at every width, up to 12288 while B has at most 12 Mi
-// elements (1088 columns at 8080: 17 against 18 us; 3232 at 6192: 23 against
-// 18, 64 at 18896: 31 against 23), and up to 32768 for one column tile (8 at
-// 33296: 24 against 34 us).
+// or a few such tiles of one column tile.  Reductions as above: up to 12288 it
+// is 0.95 - 2.8 times as fast as the split, from there 0.74 - 1.07, and up to
+// 32768 for one column tile (8 at 33296: 24 against 34 us)
 static bool few_rows_ok(int ta, int tb, size_t m, size_t n, size_t k, size_t batch)
 {
     return !ta && tb && batch == 1 && k && k % 8 == 0 && ((m <= 16 && n <= 4096) || (m <= 64 && n <= 16)) &&
-           (k <= 4096 || (k <= 12288 && n * k <= (size_t)12 << 20) || (k <= 32768 && n <= 16));
+           (k <= 12288 || (k <= 32768 && n <= 16));
 }
 
 static size_t tail_ws(int ta, int tb, size_t m, size_t n, size_t k, size_t batch)
@@ -1748,7 +1752,7 @@ extern "C" size_t pgk_gemm16_workspace_cu(int ta, int tb, size_t m, size_t n, si
 {
     if (skinny_ok(ta, tb, m, n, k, batch) || few_rows_ok(ta, tb, m, n, k, batch))
         return 0;
-    const gemm_plan pl = plan_gemm(m, n, k_inkernel(ta, tb, k), batch, cu_budget);
+    const gemm_plan pl = plan_gemm(ta, tb, m, n, k_inkernel(ta, tb, k), batch, cu_budget);
     const size_t part = pl.sp > 1 ? (((size_t)pl.sp * m * n * sizeof(float) + 255) & ~(size_t)255) : 0;
     return part + tail_ws(ta, tb, m, n, k, batch);
 }
@@ -1765,7 +1769,7 @@ extern "C" int pgk_gemm16_plan(int ta, int tb, size_t m, size_t n, size_t k, siz
             *splits = 1;
         return skinny_ok(ta, tb, m, n, k, batch) ? 4 : 9;
     }
-    const gemm_plan pl = plan_gemm(m, n, k_inkernel(ta, tb, k), batch, cu_budget);
+    const gemm_plan pl = plan_gemm(ta, tb, m, n, k_inkernel(ta, tb, k), batch, cu_budget);
     if (splits)
         *splits = pl.sp;
     return pl.tile;
@@ -1778,7 +1782,7 @@ extern "C" double pgk_gemm16_time(int ta, int tb, size_t m, size_t n, size_t k, 
     if (few_rows_ok(ta, tb, m, n, k, batch)) // B streamed once
         return (double)(n * k * 2) / 3.7e12 + 3.5e-6;
     double t = 0.0;
-    plan_gemm(m, n, k_inkernel(ta, tb, k), batch, cu_budget, &t);
+    plan_gemm(ta, tb, m, n, k_inkernel(ta, tb, k), batch, cu_budget, &t);
     return t;
 }
 
@@ -1852,7 +1856,7 @@ extern "C" int pgk_gemm16_cu(int dtype, int ta, int tb, size_t m, size_t n, size
             hipLaunchKernelGGL(k_few_rows<false>, grid, dim3(kFrWaves * 64), 0, st, kg, (int)has_epi);
         return (int)hipGetLastError();
     }
-    const gemm_plan pl = plan_gemm(m, n, kmain, batch, cu_budget);
+    const gemm_plan pl = plan_gemm(ta, tb, m, n, kmain, batch, cu_budget);
     const int sp = pl.sp > 1 ? pl.sp : 0;
     // the epilogue rides on the GEMM when one launch of the forward layout
     // finishes C, on the split-K sum when that finishes C, otherwise it is
@@ -1936,7 +1940,7 @@ extern "C" int pgk_gemm16_cu(int dtype, int ta, int tb, size_t m, size_t n, size
 // a caller whose fixed workspace cannot hold the faster plan's partials
 extern "C" int pgk_gemm16_lean_tile(int ta, int tb, size_t m, size_t n, size_t k, size_t batch)
 {
-    return m && n && batch && k && k_inkernel(ta, tb, k) == k ? ks_tile({{m, n, batch, k}}, true) : 0;
+    return m && n && batch && k && k_inkernel(ta, tb, k) == k ? ks_tile({{m, n, batch, k}}, ta && tb, true) : 0;
 }
 
 extern "C" int pgk_gemm16_lean(int dtype, int ta, int tb, size_t m, size_t n, size_t k, const uint16_t *a, size_t lda,
@@ -1977,7 +1981,7 @@ extern "C" int pgk_gemm16_pair_dw(int dtype, const pgk_gemm_desc *d, const pgk_g
     if (k_inkernel(0, 0, d->k) != d->k || k_inkernel(1, 1, w->k) != w->k ||
         skinny_ok(1, 1, w->m, w->n, w->k, w->batch))
         return PGK_GEMM_NOT_PAIRED;
-    const gemm_plan pd = plan_gemm(d->m, d->n, d->k, d->batch, cu_d), pw = plan_gemm(w->m, w->n, w->k, w->batch,
+    const gemm_plan pd = plan_gemm(0, 0, d->m, d->n, d->k, d->batch, cu_d), pw = plan_gemm(1, 1, w->m, w->n, w->k, w->batch,
                                                                                       kCUs - cu_d);
     if (pd.tile != pw.tile || pd.tile >= 5)
         return PGK_GEMM_NOT_PAIRED;
@@ -2016,7 +2020,7 @@ extern "C" int pgk_gemm16_ks_pair_tile(const pgk_gemm_desc *d, const pgk_gemm_de
     if (!d->m || !d->n || !d->k || !d->batch || !w->m || !w->n || !w->k || !w->batch || d->k % 8 ||
         skinny_ok(1, 1, w->m, w->n, w->k, w->batch))
         return 0;
-    return ks_tile({{d->m, d->n, d->batch, d->k}, {w->m, w->n, w->batch, w->k}});
+    return ks_tile({{d->m, d->n, d->batch, d->k}, {w->m, w->n, w->batch, w->k}}, false);
 }
 
 extern "C" int pgk_gemm16_ks_pair(int dtype, const pgk_gemm_desc *d, const pgk_gemm_desc *w, pgk_stream s)

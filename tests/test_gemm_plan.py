@@ -33,7 +33,7 @@ def pair_tile(k, M, K, N):
 @pytest.mark.parametrize("m,n,kk,tile", [
     (512, 512, 4096, 5), (512, 512, 65536, 0), (64, 64, 16384, 0), (72, 1080, 7520, 0),
     (512, 1024, 4096, 6), (512, 1024, 16384, 0), (1024, 1024, 4096, 8), (1024, 1024, 16384, 0),
-    (2048, 1024, 2048, 7), (2048, 1024, 12288, 0), (440, 3440, 5080, 0), (2232, 528, 2888, 0), (45, 3592, 3768, 0),
+    (2048, 1024, 2048, 7), (2048, 1024, 12288, 0), (440, 3440, 5080, 0), (2232, 528, 2888, 0), (45, 3592, 3768, 5),
 ])
 def test_long_reductions_keep_the_split_over_blocks(k, m, n, kk, tile):
     """A tile of one CU is taken up to the reduction at which eight slices of
@@ -42,8 +42,14 @@ def test_long_reductions_keep_the_split_over_blocks(k, m, n, kk, tile):
     assert got == tile if tile else got in (1, 2, 3)
 
 
+@pytest.mark.parametrize("ta,tb,kk,tile", [(1, 1, 6144, 5), (1, 1, 6152, 0), (0, 1, 10240, 5), (0, 0, 10240, 5), (0, 0, 10248, 0)])
+def test_layouts_that_read_whole_lines_hold_further(k, ta, tb, kk, tile):
+    got = k.pgk_gemm16_plan(ta, tb, 64, 640, kk, 1, 0, None)
+    assert got == tile if tile else got in (1, 2, 3)
+
+
 @pytest.mark.parametrize("m,n,kk,few", [(16, 4096, 4096, True), (16, 128, 8192, True), (64, 16, 32768, True),
-                                        (5, 3232, 6192, False), (13, 64, 18896, False), (16, 3376, 25800, False)])
+                                        (5, 3232, 6192, True), (13, 64, 18896, False), (16, 3376, 25800, False)])
 def test_few_rows_up_to_the_measured_reductions(k, m, n, kk, few):
     assert (k.pgk_gemm16_plan(0, 1, m, n, kk, 1, 0, None) == 9) == few
 
